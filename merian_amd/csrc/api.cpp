@@ -15,6 +15,7 @@
 
 #include "../../include/merian_amd.h"
 #include "bvh.h"
+#include "mrt_device.h"
 #include "mrt_kernels.h"
 #include "mrt_api_internal.h"
 
@@ -481,6 +482,8 @@ MRT_API mrt_status mrt_scene_create(mrt_ctx* c, const mrt_scene_desc* d, mrt_sce
 #undef UP
     s->ds.n_tris = uint32_t(n_tris);
     s->ds.n_geoms = d->geometry_count;
+    s->ds.layered = 0;
+    for (uint32_t k = 0; k < d->material_count; k++) s->ds.layered |= material_layered(d->materials[k]) ? 1u : 0u;
     if (st == MRT_OK) {
         const hipError_t he = hipStreamSynchronize(c->stream);
         if (he != hipSuccess) st = hip_fail(c, he, "scene upload");

@@ -21,10 +21,13 @@ namespace {
 constexpr int SHADE_BLOCK = 256;
 constexpr int SHADE_ROUNDS = 2;                          // paths per thread per tile
 constexpr int SHADE_TILE = SHADE_BLOCK * SHADE_ROUNDS;   // paths a block groups by class at once
-// Passes of at least SHADE_WIDE_PATHS paths shade tiles of SHADE_WIDE_ROUNDS paths per thread:
-// wider class groups and a more coherent continuation queue, while every resident block still
-// gets many tiles (at 1920x1080, 64 spp: 1.0 % shorter frames, 1.8 % with NEE; a 512x512
-// 4-spp pass, 1 M paths, runs 2.3 % slower with them).
+// Scenes with the full material tree (LAYERED kernels): passes of at least SHADE_WIDE_PATHS paths
+// shade tiles of SHADE_WIDE_ROUNDS paths per thread, for wider class groups and a more coherent
+// continuation queue, while every resident block still gets many tiles (at 1920x1080, 64 spp:
+// 1.0 % shorter frames, 1.8 % with NEE; a 512x512 4-spp pass, 1 M paths, runs 2.3 % slower with
+// them). The kernels without coat and sheen fit four waves per SIMD, which the wide tile's 51 KB of
+// LDS would hold at three: they take SHADE_ROUNDS always (1920x1080, 64 spp: 172.6 ms per frame
+// against 178.2 ms with wide tiles).
 constexpr int SHADE_WIDE_ROUNDS = 3;
 constexpr uint32_t SHADE_WIDE_PATHS = 1u << 23;
 constexpr float SCENE_RAY_TMAX = 1e7f;     // scene/hit.slang:8
@@ -383,7 +386,7 @@ __device__ __forceinline__ float power_heuristic(float a, float b) {
 // -----------------------------------------------------------------------------------------
 // shading points (scene.slang:312-498, hit.slang:106-147)
 
-struct ShadingPoint {
+template <bool LAYERED> struct ShadingPoint {
     f3 pos;
     uint32_t material; // material entry of a surface hit
     uint32_t enc_face_normal;
@@ -391,7 +394,7 @@ struct ShadingPoint {
     f3 emission;
     Frame frame;
     bool has_material;
-    MaterialSample mat;
+    MaterialSample<LAYERED> mat;
 };
 
 __device__ __forceinline__ f3 xyz(float4 v) { return {v.x, v.y, v.z}; }
@@ -402,8 +405,9 @@ __device__ __forceinline__ f2 uv_of(uint32_t bits) {
 // Vertex data of a hit triangle from its 64-byte shading record (DeviceScene.tri_shade: one
 // gather per hit instead of the vertex ids and three vertex records); tangents, which only
 // geometries with HasTangents use, come from the vertex records.
+template <bool LAYERED>
 __device__ __forceinline__ void shading_point(const DeviceScene& S, f3 ro, f3 rd, uint32_t gid, float bu, float bv, float ior,
-                              bool with_material, ShadingPoint& sp) {
+                              bool with_material, ShadingPoint<LAYERED>& sp) {
     float4 r0{}, r1{}, r2{}, r3{};
     uint32_t geom = 0;
     bool surface = gid != TRAVERSAL_DONE;
@@ -475,7 +479,7 @@ __device__ __forceinline__ void shading_point(const DeviceScene& S, f3 ro, f3 rd
     const mrt_material& m = S.mats[G.material_id];
     if (with_material) {
         ShadingData sd{frame, ior, front};
-        sp.mat = get_material_sample(m, sd, sp.emission, sp.frame);
+        sp.mat = get_material_sample<LAYERED>(m, sd, sp.emission, sp.frame);
     } else {
         sp.emission = material_emission(m, front);
         sp.frame = frame;
@@ -674,7 +678,8 @@ __device__ __forceinline__ void shade_sort_tile(const DeviceScene& S, const floa
 // throughput *= weight, ior follows transmission, and ShadingPoint.make_ray (hit.slang:134-146)
 // gives the next ray unless the geometric side disagrees with the transmission flag.
 // Returns whether the path continues; pdf = the sample's density.
-__device__ __forceinline__ bool bsdf_continue(const ShadingPoint& sp, f3 wi_local, f3 ng, bool wi_below, PCG& rng,
+template <bool LAYERED>
+__device__ __forceinline__ bool bsdf_continue(const ShadingPoint<LAYERED>& sp, f3 wi_local, f3 ng, bool wi_below, PCG& rng,
                                               f3& thr, float& ior, f3& next_o, f3& next_d, float& pdf) {
     const Sample s = sp.mat.sample_eval(wi_local, rng);
     if (!s.valid) return false;
@@ -710,9 +715,16 @@ __device__ __forceinline__ bool guide_eligible(const mrt_material& m) {
 // P.state once (every mode this kernel runs keeps its state in the queue). A NEE shadow ray names
 // where its contribution goes: its path's slot in the output queue (each round's continuation
 // rays are flushed before the round's shadow rays are appended) or its path's record.
-// BSDF mode fits 168 VGPRs (one spilled, no measurable cost): 3 waves per SIMD instead of 2.
-template <int MODE, int ROUNDS>
-__global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(MODE == MRT_MODE_BSDF ? 3 : 1))) void k_shade(DeviceScene S, PtArgs A, int bounce, PathBuffers P,
+// What bounds it: dependent gathers (hit -> triangle record -> material -> texels), so waves in
+// flight, and with every lobe of the material tree inlined at each use the size of the code: 37k
+// (BSDF) to 81k (guided) vector instructions and 168 to 253 registers with coat and sheen, 7k to
+// 14k and at most 128 (168 guided) without (!LAYERED), which is what most scenes take. Against the
+// full tree on the same scene: the 1920x1080 64-spp frame 180.6 -> 172.6 ms, a 957x541 16-spp NEE
+// frame 14.7 -> 12.8 ms, a 960x540 16-spp guided frame 9.2 -> 8.4 ms.
+// Waves per SIMD: 4 within 128 registers (BSDF, NEE; 3 waves: NEE 13.3 ms), 3 within 168 (guided;
+// 2 waves: 9.0 ms); the full tree keeps 3 in BSDF mode (one register spilled).
+template <int MODE, int ROUNDS, bool LAYERED>
+__global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(LAYERED ? (MODE == MRT_MODE_BSDF ? 3 : 1) : (MODE == MRT_MODE_GUIDED ? 3 : 4)))) void k_shade(DeviceScene S, PtArgs A, int bounce, PathBuffers P,
                                                        const float4* __restrict__ qo, const float4* __restrict__ qd,
                                                        const float4* __restrict__ qt, const float4* __restrict__ qr,
                                                        const uint32_t* __restrict__ count_in, float4* __restrict__ no,
@@ -766,7 +778,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(MOD
                 float ior = sa.w;
                 f3 rad{sb.x, sb.y, sb.z};
                 PCG rng{__float_as_uint(sb.w)};
-                ShadingPoint sp;
+                ShadingPoint<LAYERED> sp;
                 shading_point(S, ro, rd, gid, h4.y, h4.z, ior, bounce == 0 || !last, sp);
                 f3 emission = sp.emission;
                 if (nee && bounce > 0 && sp.env) {
@@ -903,7 +915,8 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(MOD
 // the samples of a pixel share its primary ray and gbuffer hit (render_pt.slang:99-103), so a
 // thread shades the pixel's hit once and continues every sample of the chunk from it.
 // Results per path are those of k_pt_init + k_shade<MRT_MODE_BSDF> at bounce 0.
-__global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_shade_primary(
+template <bool LAYERED>
+__global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(LAYERED ? 2 : 3))) void k_shade_primary(
     DeviceScene S, PtArgs A, const mrt_packed_hit* __restrict__ gbuffer, PathBuffers P, float4* __restrict__ no,
     float4* __restrict__ nd, float4* __restrict__ nt, float4* __restrict__ nr, uint32_t* __restrict__ count_out) {
     __shared__ float4 s_stage_o[SHADE_TILE], s_stage_d[SHADE_TILE], s_stage_t[SHADE_TILE], s_stage_r[SHADE_TILE];
@@ -917,7 +930,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(2))
         const uint32_t p = base + threadIdx.x;
         const bool valid = p < A.npix;
         uint32_t x = 0, y = 0, gid = TRAVERSAL_DONE;
-        ShadingPoint sp;
+        ShadingPoint<LAYERED> sp;
         sp.has_material = false;
         sp.emission = f3{0.f, 0.f, 0.f};
         f3 wi_local{0.f, 0.f, 1.f}, ng{0.f, 0.f, 1.f};
@@ -964,6 +977,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(2))
 // GBuffer albedo per pixel: the BSDF's directional albedo towards the camera in the material's
 // shading frame for a surface, the environment's emission for a miss (gbuffer_rt.slang:76-77,92);
 // floored at 1e-2 per channel for demodulation (gbuffer.slang:135-140).
+template <bool LAYERED>
 __global__ void k_gbuffer_albedo(DeviceScene S, mrt_camera cam, uint32_t w, uint32_t h,
                                  const mrt_packed_hit* __restrict__ gbuffer, float4* __restrict__ out, int floor) {
     const uint32_t n = w * h;
@@ -973,7 +987,7 @@ __global__ void k_gbuffer_albedo(DeviceScene S, mrt_camera cam, uint32_t w, uint
         const RayF r = camera_ray(cam, x, y, w, h);
         float bu, bv;
         const uint32_t gid = gbuffer_hit(S, gbuffer, p, bu, bv);
-        ShadingPoint sp;
+        ShadingPoint<LAYERED> sp;
         shading_point(S, r.o, r.d, gid, bu, bv, 1.f, true, sp);
         const f3 a = sp.has_material ? sp.mat.get_albedo(sp.frame.to_local(-r.d)) : sp.emission;
         out[p] = floor ? make_float4(fmaxf(a.x, 1e-2f), fmaxf(a.y, 1e-2f), fmaxf(a.z, 1e-2f), 1.f)
@@ -1071,6 +1085,7 @@ __device__ __forceinline__ void mcpg_complete(const McpgArgs& M, McpgCarry& c, f
 // Two waves per SIMD, without spills: with the path-state columns in the kernel's arguments, three
 // waves spill 15 registers and the 1080p MCPG frame takes 533 ms instead of 529 (an earlier
 // version, with fewer spills at three waves, measured the opposite: 11 % off the kernel).
+template <bool LAYERED>
 __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_shade_mcpg(
                                                             DeviceScene S, PtArgs A, McpgArgs M, int bounce,
                                                             PathBuffers P, const float4* __restrict__ qo,
@@ -1102,7 +1117,7 @@ __global__ __launch_bounds__(SHADE_BLOCK) __attribute__((amdgpu_waves_per_eu(2))
                 float ior = sa.w;
                 f3 rad{sb.x, sb.y, sb.z};
                 PCG rng{__float_as_uint(sb.w)};
-                ShadingPoint sp;
+                ShadingPoint<LAYERED> sp;
                 shading_point(S, ro, rd, gid, h4.y, h4.z, ior, bounce == 0 || !last, sp);
                 GridPos lc_here = invalid_grid_pos();
                 if (bounce == 0) {
@@ -1346,6 +1361,61 @@ hipError_t launch_trace(const DeviceScene& s, const TraceScratch& ts, const Src&
     return hipGetLastError();
 }
 
+// Launches of the shading kernels, with the full material tree (LAYERED) only for a scene that
+// has a coat or sheen lobe somewhere (DeviceScene.layered).
+template <bool LAYERED>
+void launch_shade_primary(const DeviceScene& s, const PtArgs& a, const mrt_packed_hit* gbuffer, const PathBuffers& pb,
+                          uint32_t* count_out, hipStream_t st) {
+    hipLaunchKernelGGL(k_shade_primary<LAYERED>, dim3(grid_for(a.npix, SHADE_BLOCK, MAX_BLOCKS)), dim3(SHADE_BLOCK), 0,
+                       st, s, a, gbuffer, pb, pb.q_o[1], pb.q_d[1], pb.q_t[1], pb.q_r[1], count_out);
+}
+template <int MODE, int ROUNDS, bool LAYERED>
+void launch_shade(const DeviceScene& s, const PtArgs& a, int b, const PathBuffers& pb, uint32_t* count, uint32_t* scount,
+                  hipStream_t st) {
+    const int qi = b & 1;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MODE, ROUNDS, LAYERED>),
+                       dim3(grid_for(a.n_paths, ROUNDS * SHADE_BLOCK, MAX_BLOCKS)), dim3(SHADE_BLOCK), 0, st, s, a, b, pb,
+                       pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], count, pb.q_o[qi ^ 1], pb.q_d[qi ^ 1],
+                       pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], count + 1, scount);
+}
+template <int MODE, bool LAYERED>
+void launch_shade(const DeviceScene& s, const PtArgs& a, int b, const PathBuffers& pb, uint32_t* count, uint32_t* scount,
+                  hipStream_t st) {
+    if constexpr (LAYERED) {
+        if (a.n_paths >= SHADE_WIDE_PATHS) {
+            launch_shade<MODE, SHADE_WIDE_ROUNDS, LAYERED>(s, a, b, pb, count, scount, st);
+            return;
+        }
+    }
+    launch_shade<MODE, SHADE_ROUNDS, LAYERED>(s, a, b, pb, count, scount, st);
+}
+// Shades bounce b: queue sizes count[0] (in) and count[1] (out), shadow-queue size *scount.
+template <bool LAYERED>
+void launch_shade_bounce(const DeviceScene& s, const PtArgs& a, const McpgArgs* mcpg, int b, const PathBuffers& pb,
+                         uint32_t* count, uint32_t* scount, hipStream_t st) {
+    const int qi = b & 1;
+    if (a.mode == MRT_MODE_MCPG) {
+        hipLaunchKernelGGL(k_shade_mcpg<LAYERED>, dim3(grid_for(a.n_paths, SHADE_TILE, MAX_BLOCKS)), dim3(SHADE_BLOCK), 0,
+                           st, s, a, *mcpg, b, pb, pb.q_o[qi], pb.q_d[qi], count, pb.q_o[qi ^ 1], pb.q_d[qi ^ 1],
+                           count + 1);
+    } else if (a.mode == MRT_MODE_NEE) {
+        launch_shade<MRT_MODE_NEE, LAYERED>(s, a, b, pb, count, scount, st);
+    } else if (a.mode == MRT_MODE_GUIDED) {
+        launch_shade<MRT_MODE_GUIDED, LAYERED>(s, a, b, pb, count, scount, st);
+    } else {
+        launch_shade<MRT_MODE_BSDF, LAYERED>(s, a, b, pb, count, scount, st);
+    }
+}
+void launch_albedo(const DeviceScene& s, const mrt_camera& cam, uint32_t w, uint32_t h, const mrt_packed_hit* gbuffer,
+                   float4* out, int floor, hipStream_t st) {
+    const dim3 g(grid_for(uint64_t(w) * h, 256, MAX_BLOCKS));
+    if (s.layered) {
+        hipLaunchKernelGGL(k_gbuffer_albedo<true>, g, dim3(256), 0, st, s, cam, w, h, gbuffer, out, floor);
+    } else {
+        hipLaunchKernelGGL(k_gbuffer_albedo<false>, g, dim3(256), 0, st, s, cam, w, h, gbuffer, out, floor);
+    }
+}
+
 } // namespace
 
 // ---------------------------------------------------------------------------------------------
@@ -1412,8 +1482,7 @@ hipError_t launch_gbuffer_albedo(const DeviceScene& s, const mrt_camera& cam, ui
     const uint64_t n = uint64_t(w) * h;
     if (n == 0) return hipSuccess;
     if (n > 0xFFFFFFFFull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_gbuffer_albedo, dim3(grid_for(n, 256, MAX_BLOCKS)), dim3(256), 0, st, s, cam, w, h, gbuffer,
-                       out, floor);
+    launch_albedo(s, cam, w, h, gbuffer, out, floor, st);
     return hipGetLastError();
 }
 
@@ -1465,8 +1534,7 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
     mark(-1);
     if (a.demodulate) {
         if (!pb.demod) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_gbuffer_albedo, dim3(grid_for(a.npix, 256, MAX_BLOCKS)), dim3(256), 0, st, s, a.cam,
-                           a.width, a.height, gbuffer, pb.demod, 1);
+        launch_albedo(s, a.cam, a.width, a.height, gbuffer, pb.demod, 1, st);
     }
     // [chunk][bounce] arrays: queue sizes, trace cursors, shadow-queue sizes, shadow cursors
     const uint32_t nz = n_chunks * per_chunk;
@@ -1489,8 +1557,11 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
                                cnt);
         } else if (fused_primary) {
             mark(-1);
-            hipLaunchKernelGGL(k_shade_primary, dim3(grid_for(a.npix, SHADE_BLOCK, MAX_BLOCKS)), dim3(SHADE_BLOCK), 0,
-                               st, s, a, gbuffer, pb, pb.q_o[1], pb.q_d[1], pb.q_t[1], pb.q_r[1], cnt + 1);
+            if (s.layered) {
+                launch_shade_primary<true>(s, a, gbuffer, pb, cnt + 1, st);
+            } else {
+                launch_shade_primary<false>(s, a, gbuffer, pb, cnt + 1, st);
+            }
             mark(1);
         } else {
             hipLaunchKernelGGL(k_pt_init, dim3(grid_for(a.n_paths, 256, MAX_BLOCKS)), dim3(256), 0, st, s, a, gbuffer,
@@ -1519,39 +1590,10 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
                 mark(1);
             }
             mark(-1);
-            const bool wide = a.n_paths >= SHADE_WIDE_PATHS;
-            const dim3 sg(grid_for(a.n_paths, SHADE_TILE, MAX_BLOCKS));
-            const dim3 sgw(grid_for(a.n_paths, SHADE_WIDE_ROUNDS * SHADE_BLOCK, MAX_BLOCKS));
-            if (mc) {
-                hipLaunchKernelGGL(k_shade_mcpg, sg, dim3(SHADE_BLOCK), 0, st, s, a, *mcpg, b, pb, pb.q_o[qi],
-                                   pb.q_d[qi], cnt + b, pb.q_o[qi ^ 1], pb.q_d[qi ^ 1], cnt + b + 1);
-            } else if (nee) {
-                if (wide)
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_NEE, SHADE_WIDE_ROUNDS>), sgw, dim3(SHADE_BLOCK), 0, st, s, a,
-                                       b, pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
-                else
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_NEE, SHADE_ROUNDS>), sg, dim3(SHADE_BLOCK), 0, st, s, a, b,
-                                       pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
-            } else if (guided) {
-                if (wide)
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_GUIDED, SHADE_WIDE_ROUNDS>), sgw, dim3(SHADE_BLOCK), 0, st, s, a,
-                                       b, pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
-                else
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_GUIDED, SHADE_ROUNDS>), sg, dim3(SHADE_BLOCK), 0, st, s, a, b,
-                                       pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
+            if (s.layered) {
+                launch_shade_bounce<true>(s, a, mcpg, b, pb, cnt + b, scnt + b, st);
             } else {
-                if (wide)
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_BSDF, SHADE_WIDE_ROUNDS>), sgw, dim3(SHADE_BLOCK), 0, st, s, a,
-                                       b, pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
-                else
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_shade<MRT_MODE_BSDF, SHADE_ROUNDS>), sg, dim3(SHADE_BLOCK), 0, st, s, a, b,
-                                       pb, pb.q_o[qi], pb.q_d[qi], pb.q_t[qi], pb.q_r[qi], cnt + b, pb.q_o[qi ^ 1],
-                                       pb.q_d[qi ^ 1], pb.q_t[qi ^ 1], pb.q_r[qi ^ 1], cnt + b + 1, scnt + b);
+                launch_shade_bounce<false>(s, a, mcpg, b, pb, cnt + b, scnt + b, st);
             }
             mark(1);
             if (nee && b + 1 < L && err == hipSuccess) {

@@ -603,11 +603,36 @@ struct ShadingData {
     bool front_facing;
 };
 
-// A material evaluated at a shading point (material-system.slang:64-72).
-struct MaterialSample {
+// The OpenPBR tree of a material without coat and sheen: OpenPBRBSDF with both outer weights 0, which
+// leaves the substrate, evaluated with the same operations in the same order (a Mix of weight 0
+// still renormalises its operand's sample weight, and blends its width with weight 0).
+struct UncoatedBSDF {
+    Substrate substrate;
+    MRT_HD float alpha() const { return sqrtf(pow2(sqrtf(pow2(substrate.alpha())))); }
+    MRT_HD f3 eval(f3 wi, f3 wo) const { return substrate.eval(wi, wo); }
+    MRT_HD float pdf(f3 wi, f3 wo) const { return substrate.pdf(wi, wo); }
+    MRT_HD Sample sample_eval(f3 wi, PCG& rng) const {
+        const Sample s = substrate.sample_eval(wi, rng);
+        if (!s.valid) return none_sample();
+        const f3 w = (s.weight * s.pdf) / s.pdf;
+        return make_sample(s.wo, s.pdf, (w * s.pdf) / s.pdf);
+    }
+    MRT_HD f3 get_albedo(f3 wi) const { return substrate.get_albedo(wi); }
+};
+template <bool LAYERED> struct PbrTree {
+    using type = OpenPBRBSDF;
+};
+template <> struct PbrTree<false> {
+    using type = UncoatedBSDF;
+};
+
+// A material evaluated at a shading point (material-system.slang:64-72). LAYERED: the scene has
+// a material with a coat or sheen lobe. Without one the two outer levels of the tree, whose
+// every lobe is inlined at each use, are left out of the kernels.
+template <bool LAYERED> struct MaterialSample {
     bool diffuse;
     Lambert lambert;
-    OpenPBRBSDF pbr;
+    typename PbrTree<LAYERED>::type pbr;
     float eta;
     MRT_HD Sample sample_eval(f3 wi, PCG& rng) const {
         return diffuse ? lambert.sample_eval(wi, rng) : pbr.sample_eval(wi, rng);
@@ -618,6 +643,12 @@ struct MaterialSample {
     MRT_HD f3 get_albedo(f3 wi) const { return diffuse ? lambert.get_albedo(wi) : pbr.get_albedo(wi); }
 };
 
+// Whether a material needs the LAYERED tree: a coat or sheen lobe (the feature bits that
+// get_material_sample tests).
+MRT_HD bool material_layered(const mrt_material& m) {
+    return m.model != MRT_MAT_DIFFUSE && (m.features & (MRT_PBR_CLEARCOAT | MRT_PBR_SHEEN)) != 0;
+}
+
 MRT_HD f3 material_emission(const mrt_material& m, bool front_facing) {
     if (m.model == MRT_MAT_DIFFUSE || !front_facing) return {0, 0, 0};
     return ld3(m.emission);
@@ -625,9 +656,10 @@ MRT_HD f3 material_emission(const mrt_material& m, bool front_facing) {
 
 // DiffuseMaterial::get_sample (diffuse-material.slang:163-178) and
 // OpenPBRMaterial::get_sample (openpbr-material.slang:106-209), untextured.
-MRT_HD MaterialSample get_material_sample(const mrt_material& m, const ShadingData& sd, f3& emission,
-                                          Frame& shading_frame) {
-    MaterialSample s;
+template <bool LAYERED>
+MRT_HD MaterialSample<LAYERED> get_material_sample(const mrt_material& m, const ShadingData& sd, f3& emission,
+                                                   Frame& shading_frame) {
+    MaterialSample<LAYERED> s;
     if (m.model == MRT_MAT_DIFFUSE) {
         s.diffuse = true;
         emission = {0, 0, 0};
@@ -638,8 +670,6 @@ MRT_HD MaterialSample get_material_sample(const mrt_material& m, const ShadingDa
     }
     s.diffuse = false;
     const bool has_tr = (m.features & MRT_PBR_TRANSMISSION) != 0;
-    const bool has_coat = (m.features & MRT_PBR_CLEARCOAT) != 0;
-    const bool has_sheen = (m.features & MRT_PBR_SHEEN) != 0;
     const f3 base = ld3(m.base_color);
     const float min_alpha = pow2(MIN_ROUGHNESS);
     const f2 alpha{fmaxf(m.specular_alpha[0], min_alpha), fmaxf(m.specular_alpha[1], min_alpha)};
@@ -657,22 +687,26 @@ MRT_HD MaterialSample get_material_sample(const mrt_material& m, const ShadingDa
     const Dielectric diel{OpaqueDielectric{GGX{alpha}, Lambert{base}, dielectric_f0},
                           RoughDielectric{alpha_iso, eta, tcol}, tw};
     const Substrate substrate{diel, Metal{GGX{alpha}, base}, m.metalness};
-    float cw = 0.0f, coat_alpha = min_alpha, coat_f0 = 0.0f;
-    if (has_coat) {
-        cw = m.coat_weight;
-        coat_alpha = fmaxf(m.coat_alpha, min_alpha);
-        const float ct = (m.coat_ior - 1.0f) / (m.coat_ior + 1.0f);
-        coat_f0 = ct * ct;
+    if constexpr (LAYERED) {
+        float cw = 0.0f, coat_alpha = min_alpha, coat_f0 = 0.0f;
+        if (m.features & MRT_PBR_CLEARCOAT) {
+            cw = m.coat_weight;
+            coat_alpha = fmaxf(m.coat_alpha, min_alpha);
+            const float ct = (m.coat_ior - 1.0f) / (m.coat_ior + 1.0f);
+            coat_f0 = ct * ct;
+        }
+        float sw = 0.0f, sheen_alpha = 0.0f;
+        f3 sheen_col{0.0f, 0.0f, 0.0f};
+        if (m.features & MRT_PBR_SHEEN) {
+            sw = m.sheen_weight;
+            sheen_col = ld3(m.sheen_color);
+            sheen_alpha = m.sheen_alpha;
+        }
+        s.pbr = OpenPBRBSDF{WithCoat{substrate, Coated{GGX{{coat_alpha, coat_alpha}}, substrate, coat_f0}, cw},
+                            Sheen{sheen_col, fmaxf(sheen_alpha, 1e-6f)}, sw};
+    } else {
+        s.pbr = UncoatedBSDF{substrate};
     }
-    float sw = 0.0f, sheen_alpha = 0.0f;
-    f3 sheen_col{0.0f, 0.0f, 0.0f};
-    if (has_sheen) {
-        sw = m.sheen_weight;
-        sheen_col = ld3(m.sheen_color);
-        sheen_alpha = m.sheen_alpha;
-    }
-    s.pbr = OpenPBRBSDF{WithCoat{substrate, Coated{GGX{{coat_alpha, coat_alpha}}, substrate, coat_f0}, cw},
-                        Sheen{sheen_col, fmaxf(sheen_alpha, 1e-6f)}, sw};
     emission = material_emission(m, sd.front_facing);
     s.eta = eta;
     return s;

@@ -33,6 +33,7 @@ struct DeviceScene {
     float env_to_local[9];
     uint32_t n_tris;
     uint32_t n_geoms;
+    uint32_t layered;            // some material has a coat or sheen lobe (material_layered)
     uint32_t stack_need;         // traversal stack entries the tree can need (width - 1 per level + slack)
 };
 
