@@ -79,6 +79,31 @@ __device__ __forceinline__ void grid_corners(const GuideNet& net, int l, const f
     }
 }
 
+// One of those corners: its table index and weight.
+__device__ __forceinline__ void grid_corner(uint32_t table, uint32_t res, const float pn[3], int cx, int cy, int cz,
+                                            uint32_t& idx, float& w) {
+    int ci[3];
+    float fr[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float x = pn[a] * float(res);
+        int c = int(floorf(x));
+        c = c >= int(res) ? int(res) - 1 : (c < 0 ? 0 : c);
+        ci[a] = c;
+        fr[a] = x - float(c);
+    }
+    const uint32_t ix = uint32_t(ci[0] + cx), iy = uint32_t(ci[1] + cy), iz = uint32_t(ci[2] + cz);
+    const uint64_t side = uint64_t(res) + 1;
+    const bool dense = side * side * side <= uint64_t(table);
+    const uint32_t span = table - uint32_t(side) + 1u;
+    idx = dense ? ix + uint32_t(side) * (iy + uint32_t(side) * iz)
+                : uint32_t((uint64_t((iy * 2654435761u) ^ (iz * 805459861u)) * span) >> 32) + ix;
+    const float wx = cx ? fr[0] : 1.f - fr[0];
+    const float wy = cy ? fr[1] : 1.f - fr[1];
+    const float wz = cz ? fr[2] : 1.f - fr[2];
+    w = (wx * wy) * wz;
+}
+
 __device__ __forceinline__ void normalise(const GuideNet& net, f3 p, float pn[3]) {
     pn[0] = fminf(1.f, fmaxf(0.f, (p.x - net.offset[0]) * net.scale[0]));
     pn[1] = fminf(1.f, fmaxf(0.f, (p.y - net.offset[1]) * net.scale[1]));
@@ -303,20 +328,26 @@ __global__ __launch_bounds__(GB) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // ---------------------------------------------------------------------------------------------
 // training
 
-__global__ void k_guide_sum_weights(const float4* __restrict__ rec, uint32_t n, float* __restrict__ scalars) {
-    __shared__ float part[1024];
+// Sums of the record weights by G_SUM_BLOCKS blocks, each in a fixed order; weight_sum adds them.
+// One block alone took 24 us for 65,536 records (one wave in flight per SIMD of one CU).
+__global__ __launch_bounds__(256) void k_guide_sum_weights(const float4* __restrict__ rec, uint32_t n,
+                                                           float* __restrict__ scalars) {
+    __shared__ float part[4];
     float s = 0.f;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) s += rec[3 * size_t(i)].w;
-    part[threadIdx.x] = s;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) s += rec[3 * size_t(i)].w;
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
     __syncthreads();
-    for (uint32_t w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
-        scalars[0] = part[0];
-        scalars[1] = 0.f;
+        scalars[1 + blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
+        if (blockIdx.x == 0) scalars[0] = 0.f;
     }
+}
+__device__ __forceinline__ float weight_sum(const float* __restrict__ scalars, int lane) {
+    static_assert(G_SUM_BLOCKS == 64, "one partial sum per lane");
+    float s = scalars[1 + lane];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    return s;
 }
 
 // Stores the 8 fp16 values of a B operand (features feat_of(c, g, s)) of record r.
@@ -332,62 +363,100 @@ __device__ __forceinline__ void store_operand(_Float16* base, uint32_t r, int g,
         }
 }
 
-// d(-log q)/d(outputs) of one record for lobes 4*half_ .. 4*half_+3, scaled by s; returns -log q.
-__device__ __forceinline__ float lobe_gradient(const float* o, f3 d, float s, int half_, float* g) {
-    float zmax = o[0];
-    for (int j = 1; j < G_LOBES; j++) zmax = fmaxf(zmax, o[5 * j]);
-    float e[G_LOBES], esum = 0.f;
-    for (int j = 0; j < G_LOBES; j++) {
-        e[j] = expf(o[5 * j] - zmax);
-        esum += e[j];
+// d(-log q)/d(outputs) of one record for lobes 4*half_ .. 4*half_+3 (their 20 outputs in o), scaled
+// by s; returns -log q. The two lanes of a record, lane bit 0 = half_, both call this: the softmax
+// and the mixture's density are reduced across the pair.
+__device__ __forceinline__ float lobe_gradient(const float* o, f3 d, float s, float (&g)[20]) {
+    constexpr int N = G_LOBES / 2;
+    float zmax = fmaxf(fmaxf(o[0], o[5]), fmaxf(o[10], o[15]));
+    zmax = fmaxf(zmax, __shfl_xor(zmax, 1));
+    float e[N], esum = 0.f;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        e[k] = expf(o[5 * k] - zmax);
+        esum += e[k];
     }
-    float pi[G_LOBES], kap[G_LOBES], f[G_LOBES], cm[G_LOBES], q = 0.f;
-    f3 mu[G_LOBES];
-    float len[G_LOBES];
-    bool clamped[G_LOBES];
-    for (int j = 0; j < G_LOBES; j++) {
-        pi[j] = e[j] / esum;
-        const float r = o[5 * j + 1];
-        clamped[j] = r < G_KAPPA_LOG_MIN || r > G_KAPPA_LOG_MAX;
-        kap[j] = expf(fminf(G_KAPPA_LOG_MAX, fmaxf(G_KAPPA_LOG_MIN, r)));
-        const f3 v{o[5 * j + 2], o[5 * j + 3], o[5 * j + 4]};
-        len[j] = sqrtf(dot(v, v));
-        mu[j] = len[j] > 1e-6f ? v * (1.f / len[j]) : f3{0.f, 0.f, 0.f};
-        cm[j] = dot(mu[j], d);
-        f[j] = kap[j] / (6.2831853071795864f * -expm1f(-2.f * kap[j])) * expf(kap[j] * (cm[j] - 1.f));
-        q += pi[j] * f[j];
+    esum += __shfl_xor(esum, 1);
+    float pi[N], kap[N], f[N], cm[N], len[N], q = 0.f;
+    f3 mu[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        pi[k] = e[k] / esum;
+        kap[k] = expf(fminf(G_KAPPA_LOG_MAX, fmaxf(G_KAPPA_LOG_MIN, o[5 * k + 1])));
+        const f3 v{o[5 * k + 2], o[5 * k + 3], o[5 * k + 4]};
+        len[k] = sqrtf(dot(v, v));
+        mu[k] = len[k] > 1e-6f ? v * (1.f / len[k]) : f3{0.f, 0.f, 0.f};
+        cm[k] = dot(mu[k], d);
+        f[k] = kap[k] / (6.2831853071795864f * -expm1f(-2.f * kap[k])) * expf(kap[k] * (cm[k] - 1.f));
+        q += pi[k] * f[k];
     }
-    for (int k = 0; k < 20; k++) g[k] = 0.f;
-    if (!(q > 0.f)) return 0.f;
-    for (int k = 0; k < 4; k++) {
-        const int j = 4 * half_ + k;
-        const float r = pi[j] * f[j] / q;
-        const float kk = kap[j];
-        g[5 * k] = s * (pi[j] - r);
-        const float dlogf = 1.f / kk - 2.f / expm1f(2.f * kk) + (cm[j] - 1.f);
-        g[5 * k + 1] = clamped[j] ? 0.f : s * (-r * dlogf * kk);
-        if (len[j] > 1e-6f) {
-            g[5 * k + 2] = s * (-r * kk * (d.x - cm[j] * mu[j].x) / len[j]);
-            g[5 * k + 3] = s * (-r * kk * (d.y - cm[j] * mu[j].y) / len[j]);
-            g[5 * k + 4] = s * (-r * kk * (d.z - cm[j] * mu[j].z) / len[j]);
+    q += __shfl_xor(q, 1);
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const float r = pi[k] * f[k] / q;
+        const float kk = kap[k], z = o[5 * k + 1];
+        const bool clamped = z < G_KAPPA_LOG_MIN || z > G_KAPPA_LOG_MAX;
+        const float dlogf = 1.f / kk - 2.f / expm1f(2.f * kk) + (cm[k] - 1.f);
+        const bool dir = len[k] > 1e-6f;
+        g[5 * k] = s * (pi[k] - r);
+        g[5 * k + 1] = clamped ? 0.f : s * (-r * dlogf * kk);
+        g[5 * k + 2] = dir ? s * (-r * kk * (d.x - cm[k] * mu[k].x) / len[k]) : 0.f;
+        g[5 * k + 3] = dir ? s * (-r * kk * (d.y - cm[k] * mu[k].y) / len[k]) : 0.f;
+        g[5 * k + 4] = dir ? s * (-r * kk * (d.z - cm[k] * mu[k].z) / len[k]) : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < 20; k++) g[k] = q > 0.f ? fminf(G_DOUT_CLAMP, fmaxf(-G_DOUT_CLAMP, g[k])) : 0.f;
+    return q > 0.f ? -logf(q) : 0.f;
+}
+
+// Adds the grid gradient of up to WQ records (rows of `enc`: 32 gradients at the encoding as
+// [level][feature], then the normalised position) to grid_grad.
+//
+// Eight lanes cover one cell edge along x, whose two entries are adjacent in the table: 2 x 4
+// 64-bit counters, 64 consecutive bytes. A wave's atomic instruction so touches 8 edges (four
+// edges of a cell, two levels) in 8 line segments. With one lane per (record, level) and its 32
+// counters added one instruction after the other every lane hit a line of its own, and the L2's
+// atomic request rate bound the kernel: 671 us for 65,536 records.
+__device__ __forceinline__ void scatter_grid_gradient(const GuideNet& net, const float (*enc)[48], uint32_t first,
+                                                      uint32_t n, int lane, unsigned long long* __restrict__ grid_grad) {
+    const int k = lane & 3, cx = (lane >> 2) & 1, cy = (lane >> 3) & 1, cz = (lane >> 4) & 1, lh = lane >> 5;
+    const uint32_t rows = first < n ? min(uint32_t(WQ), n - first) : 0u;
+#pragma unroll
+    for (int lp = 0; lp < G_LEVELS / 2; lp++) {
+        const int l = 2 * lp + lh;
+        const uint32_t res = lh ? net.res[2 * lp + 1] : net.res[2 * lp];
+        unsigned long long* table = grid_grad + size_t(l) * net.table * G_FEATS + k;
+#pragma unroll 2
+        for (uint32_t q = 0; q < rows; q++) {
+            const float* e = enc[q];
+            uint32_t idx;
+            float w;
+            grid_corner(net.table, res, e + G_FEATS * G_LEVELS, cx, cy, cz, idx, w);
+            const float v = w * e[G_FEATS * l + k];
+            // non-finite contributions are dropped (they would poison Adam's moments)
+            if (v != 0.f && fabsf(v) < __builtin_inff()) {
+                const float cv = fminf(fmaxf(v, -G_GRID_FX_CLAMP), G_GRID_FX_CLAMP);
+                atomicAdd(table + size_t(idx) * G_FEATS, (unsigned long long)__float2ll_rn(cv * G_GRID_FX));
+            }
         }
     }
-    for (int k = 0; k < 20; k++) g[k] = fminf(G_DOUT_CLAMP, fmaxf(-G_DOUT_CLAMP, g[k]));
-    return -logf(q);
 }
 
 // Forward and backward of BQ records per block iteration: stores every layer's input (H) and
-// output gradient (D) for the weight-gradient GEMM and adds the grid gradient.
-__global__ __launch_bounds__(GB) void k_guide_fwd_bwd(GuideNet net, const float4* __restrict__ rec, uint32_t n,
-                                                      GuideTrainBuffers B) {
+// output gradient (D) for the weight-gradient GEMM and adds the grid gradient. The backward pass
+// needs of a layer's input only which activations were positive: one bit each, instead of the
+// inputs of all layers in registers (444 registers and scratch, one wave per SIMD).
+__global__ __launch_bounds__(GB) __attribute__((amdgpu_waves_per_eu(2))) void k_guide_fwd_bwd(
+    GuideNet net, const float4* __restrict__ rec, uint32_t n, GuideTrainBuffers B) {
+    // rows of a record: the outputs, then their gradients, then the gradient at the encoding
     __shared__ float outs[4][WQ][48];
-    __shared__ float douts[4][WQ][48];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
-    const float mean_w = B.scalars[0] / float(n > 0 ? n : 1);
+    const float mean_w = weight_sum(B.scalars, lane) / float(n > 0 ? n : 1);
     for (uint32_t base = blockIdx.x * BQ; base < n; base += gridDim.x * BQ) {
-        half8_t x[5][NT][2];
+        half8_t x[NT][2];
         floatx4 acc[NT][4];
         uint32_t rid[NT];
+        uint64_t active[NT] = {}; // bit 16 k + 8 c + s: input (c, s) of layer 1 + k is positive
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             rid[t] = base + wave * WQ + t * 16 + (lane & 15);
@@ -397,19 +466,25 @@ __global__ __launch_bounds__(GB) void k_guide_fwd_bwd(GuideNet net, const float4
                 p = f3{a.x, a.y, a.z};
                 wo = f3{b.x, b.y, b.z};
             }
-            encode(net, p, wo, g, x[0][t]);
-            if (rid[t] < n) store_operand(B.H, rid[t], g, x[0][t]);
+            encode(net, p, wo, g, x[t]);
+            if (rid[t] < n) store_operand(B.H, rid[t], g, x[t]);
         }
-#pragma unroll
+#pragma unroll 1
         for (int layer = 0; layer < 4; layer++) {
-            half8_t (&xi)[NT][2] = x[layer];
-            layer_mfma<4>(net.frag_fwd, layer, xi, acc, lane);
-            relu_to_operand(acc, x[layer + 1]);
+            layer_mfma<4>(net.frag_fwd, layer, x, acc, lane);
+            relu_to_operand(acc, x);
 #pragma unroll
-            for (int t = 0; t < NT; t++)
-                if (rid[t] < n) store_operand(B.H + size_t(layer + 1) * B.cap * G_WIDTH, rid[t], g, x[layer + 1][t]);
+            for (int t = 0; t < NT; t++) {
+                uint32_t m = 0;
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int s = 0; s < 8; s++) m |= float(x[t][c][s]) > 0.f ? 1u << (8 * c + s) : 0u;
+                active[t] |= uint64_t(m) << (16 * layer);
+                if (rid[t] < n) store_operand(B.H + size_t(layer + 1) * B.cap * G_WIDTH, rid[t], g, x[t]);
+            }
         }
-        layer_mfma<3>(net.frag_fwd, 4, x[4], acc, lane);
+        layer_mfma<3>(net.frag_fwd, 4, x, acc, lane);
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -420,26 +495,31 @@ __global__ __launch_bounds__(GB) void k_guide_fwd_bwd(GuideNet net, const float4
         {
             const int qi = lane >> 1, half_ = lane & 1;
             const uint32_t i = base + wave * WQ + qi;
-            float gr[20];
-            float nlq = 0.f, s = 0.f;
-            if (i < n) {
+            const bool valid = i < n;
+            float o[20], gr[20];
+#pragma unroll
+            for (int k = 0; k < 20; k++) o[k] = outs[wave][qi][20 * half_ + k];
+            f3 dir{0.f, 0.f, 1.f};
+            float s = 0.f;
+            if (valid) {
                 const float4 a = rec[3 * size_t(i)], c = rec[3 * size_t(i) + 2];
                 s = mean_w > 0.f ? fminf(G_WEIGHT_SCALE_MAX, a.w / mean_w) : 0.f;
-                nlq = lobe_gradient(outs[wave][qi], f3{c.x, c.y, c.z}, s, half_, gr);
-            } else {
-                for (int k = 0; k < 20; k++) gr[k] = 0.f;
+                dir = f3{c.x, c.y, c.z};
             }
-            for (int k = 0; k < 20; k++) douts[wave][qi][20 * half_ + k] = gr[k];
+            const float nlq = lobe_gradient(o, dir, s, gr);
+            __syncthreads(); // every output is in registers: the rows now take the gradients
+#pragma unroll
+            for (int k = 0; k < 20; k++) outs[wave][qi][20 * half_ + k] = valid ? gr[k] : 0.f;
             if (half_ == 1)
-                for (int k = 40; k < 48; k++) douts[wave][qi][k] = 0.f;
+#pragma unroll
+                for (int k = 40; k < 48; k++) outs[wave][qi][k] = 0.f;
             // loss: one lane per record, one atomic per wave
-            float l = (half_ == 0 && i < n) ? s * nlq : 0.f;
+            float l = (half_ == 0 && valid) ? s * nlq : 0.f;
             for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-            if (lane == 0) atomicAdd(B.scalars + 1, l);
+            if (lane == 0) atomicAdd(B.scalars, l);
         }
         __syncthreads();
         // gradient at the outputs as B operand (features >= 48 are zero)
-        half8_t d[NT][2];
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -447,53 +527,44 @@ __global__ __launch_bounds__(GB) void k_guide_fwd_bwd(GuideNet net, const float4
 #pragma unroll
                 for (int s = 0; s < 8; s++) {
                     const int fo = feat_of(c, g, s);
-                    d[t][c][s] = _Float16(fo < 48 ? douts[wave][t * 16 + (lane & 15)][fo] : 0.f);
+                    x[t][c][s] = _Float16(fo < 48 ? outs[wave][t * 16 + (lane & 15)][fo] : 0.f);
                 }
-#pragma unroll
+#pragma unroll 1
         for (int layer = 4; layer >= 0; layer--) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
-                if (rid[t] < n) store_operand(B.D + size_t(layer) * B.cap * G_WIDTH, rid[t], g, d[t]);
-            layer_mfma<4>(net.frag_bwd, layer, d, acc, lane); // acc = W^T d: gradient at the layer's input
+                if (rid[t] < n) store_operand(B.D + size_t(layer) * B.cap * G_WIDTH, rid[t], g, x[t]);
+            layer_mfma<4>(net.frag_bwd, layer, x, acc, lane); // acc = W^T d: gradient at the layer's input
             if (layer > 0) {
 #pragma unroll
-                for (int t = 0; t < NT; t++)
+                for (int t = 0; t < NT; t++) {
+                    const uint32_t m = uint32_t(active[t] >> (16 * (layer - 1)));
 #pragma unroll
                     for (int c = 0; c < 2; c++)
 #pragma unroll
                         for (int s = 0; s < 8; s++)
-                            d[t][c][s] = _Float16(float(x[layer][t][c][s]) > 0.f ? acc[t][2 * c + (s >> 2)][s & 3] : 0.f);
-            }
-        }
-        // acc = gradient at the encoding: in-tile 0 holds features 4g+r (level g), in-tile 1
-        // holds 16+4g+r (level 4+g)
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            if (rid[t] >= n) continue;
-            const float4 a = rec[3 * size_t(rid[t])];
-            float pn[3];
-            normalise(net, f3{a.x, a.y, a.z}, pn);
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int l = slot_level(g, h);
-                uint32_t idx[8];
-                float w[8];
-                grid_corners(net, l, pn, idx, w);
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    unsigned long long* gg = B.grid_grad + (size_t(l) * net.table + idx[c]) * G_FEATS;
-#pragma unroll
-                    for (int k = 0; k < G_FEATS; k++) {
-                        const float v = w[c] * acc[t][h][k];
-                        // non-finite contributions are dropped (they would poison Adam's moments)
-                        if (v != 0.f && fabsf(v) < __builtin_inff()) {
-                            const float cv = fminf(fmaxf(v, -G_GRID_FX_CLAMP), G_GRID_FX_CLAMP);
-                            atomicAdd(gg + k, (unsigned long long)__float2ll_rn(cv * G_GRID_FX));
-                        }
-                    }
+                            x[t][c][s] = _Float16((m >> (8 * c + s)) & 1u ? acc[t][2 * c + (s >> 2)][s & 3] : 0.f);
                 }
             }
         }
+        // acc = gradient at the encoding: in-tile 0 holds features 4g+r (level g), in-tile 1
+        // holds 16+4g+r (level 4+g). It goes through LDS (the output rows, read for the last time
+        // above) so that the lanes of one atomic instruction cover whole cell edges.
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            float* o = outs[wave][t * 16 + (lane & 15)];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int k = 0; k < G_FEATS; k++) o[G_FEATS * slot_level(g, h) + k] = acc[t][h][k];
+            if (g == 0 && rid[t] < n) {
+                const float4 a = rec[3 * size_t(rid[t])];
+                normalise(net, f3{a.x, a.y, a.z}, o + G_FEATS * G_LEVELS);
+            }
+        }
+        __syncthreads();
+        scatter_grid_gradient(net, outs[wave], base + wave * WQ, n, lane, B.grid_grad);
     }
 }
 
@@ -542,13 +613,26 @@ __global__ __launch_bounds__(GB) void k_guide_wgrad(GuideTrainBuffers B, uint32_
         for (int r = 0; r < 4; r++) P[(16 * wave + 4 * g + r) * G_WIDTH + 16 * it + (lane & 15)] = acc[it][r];
 }
 
-__global__ void k_guide_reduce_wgrad(GuideTrainBuffers B, float* __restrict__ dW) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= uint32_t(G_LAYERS * G_WIDTH * G_WIDTH)) return;
-    const uint32_t layer = e / (G_WIDTH * G_WIDTH), k = e % (G_WIDTH * G_WIDTH);
+// Sum over the blocks' partials of weight element e, by the four waves of a block of GB threads
+// (64 elements per block; wave w takes every fourth partial from w on); valid in wave 0. Every
+// thread of the block calls this.
+constexpr int WSUM_ELEMS = 64;
+__device__ __forceinline__ float wgrad_sum(const GuideTrainBuffers& B, uint32_t e) {
+    __shared__ float part[4][WSUM_ELEMS];
+    const uint32_t layer = e / (G_WIDTH * G_WIDTH), k = e % (G_WIDTH * G_WIDTH), wave = threadIdx.x >> 6;
+    const float* p = B.partials + size_t(layer) * B.kblocks * G_WIDTH * G_WIDTH + k;
     float s = 0.f;
-    for (uint32_t kb = 0; kb < B.kblocks; kb++) s += B.partials[(size_t(layer) * B.kblocks + kb) * G_WIDTH * G_WIDTH + k];
-    dW[e] = s;
+    for (uint32_t kb = wave; kb < B.kblocks; kb += 4) s += p[size_t(kb) * G_WIDTH * G_WIDTH];
+    part[wave][threadIdx.x & 63] = s;
+    __syncthreads();
+    const uint32_t c = threadIdx.x & 63;
+    return (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+}
+
+__global__ __launch_bounds__(GB) void k_guide_reduce_wgrad(GuideTrainBuffers B, float* __restrict__ dW) {
+    const uint32_t e = blockIdx.x * WSUM_ELEMS + (threadIdx.x & 63);
+    const float s = wgrad_sum(B, e);
+    if (threadIdx.x < WSUM_ELEMS) dW[e] = s;
 }
 
 // Fragment positions of weight W_layer[o][i]: forward (A = W) and backward (A = W^T).
@@ -565,16 +649,14 @@ __device__ __forceinline__ void frag_positions(int layer, int o, int i, uint32_t
     }
 }
 
-__global__ void k_guide_adam_w(GuideParams p, GuideTrainBuffers B, float lr, float scale, float bc1, float bc2,
-                               int update) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= uint32_t(G_LAYERS * G_WIDTH * G_WIDTH)) return;
+__global__ __launch_bounds__(GB) void k_guide_adam_w(GuideParams p, GuideTrainBuffers B, float lr, float scale,
+                                                     float bc1, float bc2, int update) {
+    const uint32_t e = blockIdx.x * WSUM_ELEMS + (threadIdx.x & 63);
+    const float gsum = update ? wgrad_sum(B, e) : 0.f;
+    if (threadIdx.x >= WSUM_ELEMS) return;
     const int layer = int(e / (G_WIDTH * G_WIDTH)), o = int((e / G_WIDTH) % G_WIDTH), i = int(e % G_WIDTH);
     float w = p.w[e];
     if (update && !(layer == G_LAYERS - 1 && o >= G_OUT)) {
-        float gsum = 0.f;
-        for (uint32_t kb = 0; kb < B.kblocks; kb++)
-            gsum += B.partials[(size_t(layer) * B.kblocks + kb) * G_WIDTH * G_WIDTH + uint32_t(o) * G_WIDTH + i];
         const float gr = gsum * scale;
         const float m = 0.9f * p.w_m[e] + 0.1f * gr;
         const float v = 0.99f * p.w_v[e] + 0.01f * gr * gr;
@@ -666,7 +748,7 @@ hipError_t launch_guide_forward(const GuideNet& net, const float4* pos, const fl
 hipError_t launch_guide_gradient(const GuideNet& net, const float4* records, uint32_t n, GuideTrainBuffers& b,
                                  hipStream_t st) {
     if (n > b.cap) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_guide_sum_weights, dim3(1), dim3(1024), 0, st, records, n, b.scalars);
+    hipLaunchKernelGGL(k_guide_sum_weights, dim3(G_SUM_BLOCKS), dim3(256), 0, st, records, n, b.scalars);
     if (n == 0) return hipGetLastError();
     hipLaunchKernelGGL(k_guide_fwd_bwd, dim3(blocks_for(n, BQ, 1024)), dim3(GB), 0, st, net, records, n, b);
     const uint32_t kb = (n + G_WGRAD_RECORDS - 1) / G_WGRAD_RECORDS;
@@ -678,13 +760,13 @@ hipError_t launch_guide_gradient(const GuideNet& net, const float4* records, uin
 }
 
 hipError_t launch_guide_reduce_wgrad(const GuideTrainBuffers& b, float* dW, hipStream_t st) {
-    hipLaunchKernelGGL(k_guide_reduce_wgrad, dim3((G_LAYERS * G_WIDTH * G_WIDTH + 255) / 256), dim3(256), 0, st, b, dW);
+    hipLaunchKernelGGL(k_guide_reduce_wgrad, dim3(G_LAYERS * G_WIDTH * G_WIDTH / WSUM_ELEMS), dim3(GB), 0, st, b, dW);
     return hipGetLastError();
 }
 
 hipError_t launch_guide_adam(const GuideParams& p, const GuideTrainBuffers& b, float lr, float scale, float bc1,
                              float bc2, hipStream_t st) {
-    hipLaunchKernelGGL(k_guide_adam_w, dim3((G_LAYERS * G_WIDTH * G_WIDTH + 255) / 256), dim3(256), 0, st, p, b, lr,
+    hipLaunchKernelGGL(k_guide_adam_w, dim3(G_LAYERS * G_WIDTH * G_WIDTH / WSUM_ELEMS), dim3(GB), 0, st, p, b, lr,
                        scale, bc1, bc2, 1);
     hipLaunchKernelGGL(k_guide_adam_grid, dim3(blocks_for(p.grid_count, 256, 8192)), dim3(256), 0, st, p, b.grid_grad,
                        lr, scale, bc1, bc2, 1);
@@ -693,7 +775,7 @@ hipError_t launch_guide_adam(const GuideParams& p, const GuideTrainBuffers& b, f
 
 hipError_t launch_guide_pack(const GuideParams& p, hipStream_t st) {
     GuideTrainBuffers none{};
-    hipLaunchKernelGGL(k_guide_adam_w, dim3((G_LAYERS * G_WIDTH * G_WIDTH + 255) / 256), dim3(256), 0, st, p, none,
+    hipLaunchKernelGGL(k_guide_adam_w, dim3(G_LAYERS * G_WIDTH * G_WIDTH / WSUM_ELEMS), dim3(GB), 0, st, p, none,
                        0.f, 0.f, 1.f, 1.f, 0);
     hipLaunchKernelGGL(k_guide_adam_grid, dim3(blocks_for(p.grid_count, 256, 8192)), dim3(256), 0, st, p, nullptr,
                        0.f, 0.f, 1.f, 1.f, 0);

@@ -270,7 +270,7 @@ MRT_API mrt_status mrt_guide_create(mrt_ctx* c, mrt_scene* s, const mrt_guide_co
     g->P.grid = galloc<_Float16>(c, g, ng, &st);
     g->P.grid_count = ng;
     g->T.grid_grad = galloc<unsigned long long>(c, g, ng, &st);
-    g->T.scalars = galloc<float>(c, g, 4, &st);
+    g->T.scalars = galloc<float>(c, g, 1 + G_SUM_BLOCKS, &st);
     g->dW = galloc<float>(c, g, nw, &st);
     g->grec = galloc<float4>(c, g, size_t(5) * cfg.max_records, &st);
     g->gtrain = galloc<float4>(c, g, size_t(3) * cfg.max_records, &st);
@@ -412,18 +412,18 @@ MRT_API mrt_status mrt_guide_gradient(mrt_ctx* c, mrt_guide* g, const float* rec
     hipError_t e = hipMemsetAsync(g->T.grid_grad, 0, gbytes, c->stream);
     if (e == hipSuccess) e = launch_guide_gradient(g->net, g->host_records, n, tb, c->stream);
     if (e == hipSuccess) e = launch_guide_reduce_wgrad(tb, g->dW, c->stream);
-    float sc[2] = {0.f, 0.f};
+    float loss_sum = 0.f;
     std::vector<unsigned long long> fx(d_grid ? g->P.grid_count : 0);
     if (e == hipSuccess && d_weights)
         e = hipMemcpyAsync(d_weights, g->dW, size_t(G_LAYERS) * G_WIDTH * G_WIDTH * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess && d_grid) e = hipMemcpyAsync(fx.data(), g->T.grid_grad, gbytes, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(sc, g->T.scalars, 8, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&loss_sum, g->T.scalars, 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     // leave the gradient accumulator cleared for training
     if (e == hipSuccess) e = hipMemsetAsync(g->T.grid_grad, 0, gbytes, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "mrt_guide_gradient");
     for (size_t k = 0; k < fx.size(); k++) d_grid[k] = float(double((long long)fx[k]) / double(G_GRID_FX));
-    if (loss) *loss = sc[1] / float(n);
+    if (loss) *loss = loss_sum / float(n);
     return MRT_OK;
 }
 
@@ -443,11 +443,11 @@ MRT_API mrt_status mrt_guide_train(mrt_ctx* c, mrt_guide* g, const float* record
         st = train_step(c, g, g->host_records + 3 * size_t(off), last, c->stream);
     }
     if (st != MRT_OK) return st;
-    float sc[2] = {0.f, 0.f};
-    hipError_t e = hipMemcpyAsync(sc, g->T.scalars, 8, hipMemcpyDeviceToHost, c->stream);
+    float loss_sum = 0.f;
+    hipError_t e = hipMemcpyAsync(&loss_sum, g->T.scalars, 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "mrt_guide_train");
-    if (loss) *loss = sc[1] / float(last);
+    if (loss) *loss = loss_sum / float(last);
     return MRT_OK;
 }
 

@@ -122,10 +122,14 @@ struct GuideTrainBuffers {
     // [level][table][G_FEATS] grid gradient as 64-bit fixed point (G_GRID_FX units): integer
     // atomics sum it exactly, so the sum does not depend on the order the records arrive in
     unsigned long long* grid_grad;
-    float* scalars;    // [0] weight sum, [1] loss sum
+    float* scalars;    // [0] loss sum, [1 ..] weight sums of G_SUM_BLOCKS blocks
     uint32_t cap, kblocks;
 };
-constexpr uint32_t G_WGRAD_RECORDS = 2048; // records per weight-gradient block
+// Records per weight-gradient block: a block stages 32 at a time and waits for memory each time, so
+// the chip needs many short blocks (65,536 records, 5 layers: 640; with 2048 records per block,
+// 160 blocks, the kernel took 60 us)
+constexpr uint32_t G_WGRAD_RECORDS = 512;
+constexpr int G_SUM_BLOCKS = 64;           // blocks of the weight sum
 constexpr float G_GRID_FX = 16777216.f;      // grid-gradient fixed point: 2^24 units per 1
 constexpr float G_GRID_FX_CLAMP = 4096.f;    // one corner's contribution, as the output gradients
 
