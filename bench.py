@@ -28,7 +28,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Mpath-segments/s at 1080p; equal-time relMSE guided vs plain; p99 job latency"
 HBM_PEAK_GBS = 8000.0
-NODE_BYTES = {4: 128, 8: 80}  # BVH4Node (fp32 boxes), BVH8Node (8-bit quantized boxes)
+NODE_BYTES = {4: 48, 8: 80}  # BVH4Node, BVH8Node (8-bit quantized boxes)
 TRI_BYTES = 48        # TriRecord
 RAY_IO_BYTES = 32 + 16  # queued ray in, hit out
 # HBM bytes per dispatch of the intersect kernel, measured with rocprofv3 FETCH_SIZE / WRITE_SIZE

@@ -231,7 +231,7 @@ typedef struct mrt_pt_stats {
     float ms_total;                 /* device time of the whole frame */
     uint32_t trace_launches;        /* intersect-kernel launches of the frame */
     uint32_t _pad;
-    uint64_t node_visits;           /* BVH4 node visits (count_traversal only) */
+    uint64_t node_visits;           /* BVH node visits (count_traversal only) */
     uint64_t triangle_tests;        /* ray-triangle tests (count_traversal only) */
 } mrt_pt_stats;
 
@@ -349,7 +349,7 @@ typedef struct mrt_tuning {
     uint32_t grid_percent;    /* persistent traversal grid, percent of the resident blocks */
     uint32_t bvh_max_leaf;    /* triangles per BVH leaf, 1..8 */
     float bvh_traversal_cost; /* SAH cost of a node visit relative to a triangle test */
-    uint32_t bvh_width;       /* BVH node width: 4 (full-precision boxes, 128-byte nodes) or 8
+    uint32_t bvh_width;       /* BVH node width: 4 (8-bit quantised boxes, 48-byte nodes) or 8
                                  (8-bit quantised boxes, 80-byte nodes) */
     float ms_per_frame;       /* frame time measured for these settings (mrt_tune) */
     uint32_t leaf_lanes;      /* lanes of 64 left with nothing but a postponed leaf before a

@@ -126,7 +126,7 @@ mrt_status ensure_path_buffers(mrt_ctx* c, uint64_t paths, uint64_t npix, uint64
 
 // Global part of the traversal stacks, sized for the deepest scene traced so far.
 mrt_status ensure_trace_scratch(mrt_ctx* c, const mrt_scene* s) {
-    const uint32_t need = s->ds.stack_need > uint32_t(TRACE_LDS_STACK) ? s->ds.stack_need - TRACE_LDS_STACK : 1u;
+    const uint32_t need = trace_ovf_entries(s->ds.stack_need);
     TraceScratch& t = c->trace;
     if (t.work && t.entries >= need) return MRT_OK;
     if (t.ovf) dev_free(c, t.ovf);
@@ -425,7 +425,7 @@ MRT_API mrt_status mrt_scene_create(mrt_ctx* c, const mrt_scene_desc* d, mrt_sce
         }
     }
     const mrt_tuning defaults = mrt_scene{}.tuning;
-    const BVH4 bvh = build_bvh4(v0.data(), e1.data(), e2.data(), flags.data(), uint32_t(n_tris), 0,
+    BVH4 bvh = build_bvh4(v0.data(), e1.data(), e2.data(), flags.data(), uint32_t(n_tris), 0,
                                 int(defaults.bvh_max_leaf), defaults.bvh_traversal_cost);
     mrt_scene* s = new mrt_scene();
     if (n_tris) {
@@ -440,7 +440,9 @@ MRT_API mrt_status mrt_scene_create(mrt_ctx* c, const mrt_scene_desc* d, mrt_sce
                 s->bbox_max[k] = std::max(s->bbox_max[k], std::max(a, std::max(b, cc)));
             }
     }
+    bvh.tris.resize(bvh.tris.size() + TRI_PADDING);
     s->ds.stack_need = 3u * bvh.depth + 4u;
+    s->ds.dir_min = bvh_dir_min(bvh.max_exp);
     s->ds.width = 4;
     s->ds.nodes8 = nullptr;
     s->n_tris = n_tris;

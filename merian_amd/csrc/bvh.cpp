@@ -1,4 +1,4 @@
-// Binned-SAH BVH2 build, collapsed into the 128-byte BVH4 layout of bvh.h.
+// Binned-SAH BVH2 build, collapsed into the quantised BVH4 and BVH8 layouts of bvh.h.
 //
 // The reference leaves BVH construction to the Vulkan driver (PreferFastTrace for static mesh
 // groups, src/merian-shaders/scene/scene.cpp:1116-1123). This builder is the project's own:
@@ -177,64 +177,6 @@ void padded(const AABB& b, float mag, float lo[3], float hi[3]) {
     }
 }
 
-struct Collapser {
-    const std::vector<Node2>& n2;
-    BVH4& out;
-    float mag;
-
-    uint32_t collapse(int32_t ni, uint32_t depth) {
-        int32_t kids[4];
-        int nk = 0;
-        const Node2& root = n2[ni];
-        kids[nk++] = root.left;
-        kids[nk++] = root.right;
-        while (nk < 4) {
-            int best = -1;
-            float best_area = -1.f;
-            for (int i = 0; i < nk; i++) {
-                const Node2& c = n2[kids[i]];
-                if (c.left >= 0 && c.box.area() > best_area) {
-                    best_area = c.box.area();
-                    best = i;
-                }
-            }
-            if (best < 0) break;
-            const Node2& c = n2[kids[best]];
-            kids[best] = c.left;
-            kids[nk++] = c.right;
-        }
-        const uint32_t me = uint32_t(out.nodes.size());
-        out.nodes.emplace_back();
-        out.depth = std::max(out.depth, depth);
-        BVH4Node node;
-        std::memset(&node, 0, sizeof(node));
-        for (int i = 0; i < 4; i++) {
-            if (i >= nk) {
-                node.lox[i] = node.loy[i] = node.loz[i] = 1e30f;
-                node.hix[i] = node.hiy[i] = node.hiz[i] = -1e30f;
-                node.entry[i] = EMPTY_ENTRY;
-                continue;
-            }
-            const Node2& c = n2[kids[i]];
-            float lo[3], hi[3];
-            padded(c.box, mag, lo, hi);
-            node.lox[i] = lo[0];
-            node.loy[i] = lo[1];
-            node.loz[i] = lo[2];
-            node.hix[i] = hi[0];
-            node.hiy[i] = hi[1];
-            node.hiz[i] = hi[2];
-            if (c.left < 0) {
-                node.entry[i] = leaf_entry(c.first, c.count);
-            } else {
-                node.entry[i] = collapse(kids[i], depth + 1);
-            }
-        }
-        out.nodes[me] = node;
-        return me;
-    }
-};
-
 float down(double v) {
     float f = float(v);
     if (double(f) > v) f = std::nextafter(f, -INFINITY);
@@ -320,7 +262,18 @@ struct Quant {
     int e[3];
 };
 
-Quant node_grid(const float (*lo)[3], const float (*hi)[3], int nk) {
+// Rounds a grid origin down to the 24 bits a BVH4 node keeps of it.
+float origin24(float v) {
+    uint32_t b;
+    std::memcpy(&b, &v, 4);
+    if ((b & 0x80000000u) && (b & ~BVH4_ORIGIN_MASK)) b += 0x100u;
+    b &= BVH4_ORIGIN_MASK;
+    std::memcpy(&v, &b, 4);
+    return v;
+}
+
+// width: the children per node of the tree, whose nodes keep the origin in 24 (4) or 32 (8) bits.
+Quant node_grid(const float (*lo)[3], const float (*hi)[3], int nk, int width) {
     Quant q;
     for (int a = 0; a < 3; a++) {
         float mn = FLT_MAX, mx = -FLT_MAX;
@@ -328,11 +281,12 @@ Quant node_grid(const float (*lo)[3], const float (*hi)[3], int nk) {
             mn = std::min(mn, lo[k][a]);
             mx = std::max(mx, hi[k][a]);
         }
+        if (width == 4) mn = origin24(mn);
         q.p[a] = mn;
         const double ext = double(mx) - double(mn);
         int e = -126;
         if (ext > 0) {
-            e = int(std::ceil(std::log2(ext / 250.0)));
+            if (std::frexp(ext / 250.0, &e) == 0.5) e--; // ceil(log2(ext / 250))
             while (std::ldexp(250.0, e) < ext) e++;
         }
         q.e[a] = std::max(-126, std::min(127, e));
@@ -354,12 +308,14 @@ uint8_t quant_hi(float v, float p, float s) {
     return uint8_t(qi);
 }
 
-struct Collapser8 {
+template <class Tree> struct Collapser {
+    using Node = typename decltype(Tree::nodes)::value_type;
+    static constexpr int W = sizeof(Node::code);
     const std::vector<Node2>& n2;
     const std::vector<uint32_t>& idx;
     const float *v0, *e1, *e2;
     const uint32_t* flags;
-    BVH8& out;
+    Tree& out;
     float mag;
 
     // Places the node's children in slots by corner: slot bit a set = the child lies toward the
@@ -405,33 +361,53 @@ struct Collapser8 {
         }
     }
 
+    static void set_grid(BVH8Node& n, const Quant& g) {
+        n.px = g.p[0];
+        n.py = g.p[1];
+        n.pz = g.p[2];
+        n.ex = int8_t(g.e[0]);
+        n.ey = int8_t(g.e[1]);
+        n.ez = int8_t(g.e[2]);
+    }
+    static void set_grid(BVH4Node& n, const Quant& g) {
+        uint32_t* p[3] = {&n.px, &n.py, &n.pz};
+        for (int a = 0; a < 3; a++) {
+            std::memcpy(p[a], &g.p[a], 4);
+            *p[a] |= uint32_t(uint8_t(int8_t(g.e[a])));
+        }
+    }
+
     // fills out.nodes[me] from BVH2 node ni (or a lone leaf when ni is a leaf)
     void emit(int32_t ni, uint32_t me, uint32_t depth) {
         out.depth = std::max(out.depth, depth);
-        int32_t kids[8];
+        int32_t kids[W];
         int nk;
         if (n2[ni].left < 0) {
             kids[0] = ni;
             nk = 1;
         } else {
-            nk = gather_children(n2, ni, 8, kids);
+            nk = gather_children(n2, ni, W, kids);
         }
-        int32_t sk[8];
-        assign_slots(kids, nk, sk);
-        float lo[8][3], hi[8][3];
-        for (int k = 0; k < nk; k++) padded(n2[kids[k]].box, mag, lo[k], hi[k]);
-        const Quant g = node_grid(lo, hi, nk);
-        BVH8Node node;
+        int32_t sk[W];
+        if constexpr (W == 8) {
+            assign_slots(kids, nk, sk);
+        } else {
+            for (int s = 0; s < W; s++) sk[s] = s < nk ? kids[s] : -1;
+        }
+        float lo[W][3], hi[W][3];
+        for (int s = 0, k = 0; s < W; s++)
+            if (sk[s] >= 0) {
+                padded(n2[sk[s]].box, mag, lo[k], hi[k]);
+                k++;
+            }
+        const Quant g = node_grid(lo, hi, nk, W);
+        Node node;
         std::memset(&node, 0, sizeof(node));
-        node.px = g.p[0];
-        node.py = g.p[1];
-        node.pz = g.p[2];
-        node.ex = int8_t(g.e[0]);
-        node.ey = int8_t(g.e[1]);
-        node.ez = int8_t(g.e[2]);
+        set_grid(node, g);
+        out.max_exp = std::max(out.max_exp, std::max(g.e[0], std::max(g.e[1], g.e[2])));
         uint8_t* qlo[3] = {node.qlox, node.qloy, node.qloz};
         uint8_t* qhi[3] = {node.qhix, node.qhiy, node.qhiz};
-        for (int k = 0; k < 8; k++)
+        for (int k = 0; k < W; k++)
             for (int a = 0; a < 3; a++) {
                 qlo[a][k] = 255;
                 qhi[a][k] = 0;
@@ -442,24 +418,23 @@ struct Collapser8 {
         node.child_base = uint32_t(out.nodes.size());
         out.nodes.resize(out.nodes.size() + size_t(n_inner));
         node.tri_base = uint32_t(out.tris.size());
-        std::memset(node.code, BVH8_EMPTY, 8);
+        std::memset(node.code, BVH8_EMPTY, W);
+        const float step[3] = {std::ldexp(1.0f, g.e[0]), std::ldexp(1.0f, g.e[1]), std::ldexp(1.0f, g.e[2])};
         uint32_t rank = 0;
-        for (int s = 0; s < 8; s++) {
+        for (int s = 0, k = 0; s < W; s++) {
             if (sk[s] < 0) continue;
             const Node2& c = n2[sk[s]];
-            float clo[3], chi[3];
-            padded(c.box, mag, clo, chi);
             for (int a = 0; a < 3; a++) {
-                const float sc = std::ldexp(1.0f, g.e[a]);
-                qlo[a][s] = quant_lo(clo[a], g.p[a], sc);
-                qhi[a][s] = quant_hi(chi[a], g.p[a], sc);
+                qlo[a][s] = quant_lo(lo[k][a], g.p[a], step[a]);
+                qhi[a][s] = quant_hi(hi[k][a], g.p[a], step[a]);
             }
+            k++;
             if (c.left >= 0) {
-                node.inner_mask |= uint8_t(1u << s);
+                if constexpr (W == 8) node.inner_mask |= uint8_t(1u << s);
                 node.code[s] = uint8_t(BVH8_INNER + rank++);
             } else {
                 const uint32_t off = uint32_t(out.tris.size()) - node.tri_base;
-                node.code[s] = uint8_t(off << 3 | (c.count - 1u)); // count in [1, BVH8_MAX_LEAF]
+                node.code[s] = uint8_t(off << 3 | (c.count - 1u)); // count in [1, MAX_LEAF] ([1, BVH8_MAX_LEAF])
                 for (uint32_t t = 0; t < c.count; t++) {
                     out.tris.emplace_back();
                     set_record(out.tris.back(), idx[c.first + t], v0, e1, e2, flags);
@@ -468,111 +443,52 @@ struct Collapser8 {
         }
         out.nodes[me] = node;
         uint32_t slot = node.child_base;
-        for (int s = 0; s < 8; s++)
+        for (int s = 0; s < W; s++)
             if (sk[s] >= 0 && n2[sk[s]].left >= 0) emit(sk[s], slot++, depth + 1);
     }
 };
 
-} // namespace
-
-BVH4 build_bvh4(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n,
-                int threads, int max_leaf, float traversal_cost) {
-    if (threads <= 0) threads = int(std::max(1u, std::thread::hardware_concurrency()));
-    Prepared pr = prepare(v0, e1, e2, n);
-    const std::vector<Prim>& prims = pr.prims;
-    std::vector<uint32_t>& order = pr.order;
-    const float mag = pr.mag;
-    BVH4 out;
-    const uint32_t m = uint32_t(order.size());
-    Builder bld(prims, std::move(order), threads);
-    bld.max_leaf = uint32_t(std::min(std::max(max_leaf, 1), MAX_LEAF));
-    bld.traversal_cost = traversal_cost > 0.f ? traversal_cost : 1.0f;
-    if (m > 0) bld.build(0, 0, m, 0);
-    // triangle records in leaf order
-    out.tris.resize(m);
-    for (uint32_t k = 0; k < m; k++) {
-        const uint32_t i = bld.idx[k];
-        TriRecord& t = out.tris[k];
-        for (int c = 0; c < 3; c++) {
-            t.a[c] = v0[3 * i + c];
-            t.b[c] = e1[3 * i + c];
-            t.c[c] = e2[3 * i + c];
-        }
-        std::memcpy(&t.a[3], &i, 4);
-        std::memcpy(&t.b[3], &flags[i], 4);
-        t.c[3] = 0.f;
-    }
-    if (m == 0) {
-        // empty scene: one node with four empty children
-        BVH4Node node;
-        std::memset(&node, 0, sizeof(node));
-        for (int i = 0; i < 4; i++) {
-            node.lox[i] = node.loy[i] = node.loz[i] = 1e30f;
-            node.hix[i] = node.hiy[i] = node.hiz[i] = -1e30f;
-            node.entry[i] = EMPTY_ENTRY;
-        }
-        out.nodes.push_back(node);
-        out.depth = 1;
-        return out;
-    }
-    const Node2& root = bld.nodes[0];
-    if (root.left < 0) {
-        // single leaf: wrap it in a root node with one leaf child
-        BVH4Node node;
-        std::memset(&node, 0, sizeof(node));
-        for (int i = 0; i < 4; i++) {
-            node.lox[i] = node.loy[i] = node.loz[i] = 1e30f;
-            node.hix[i] = node.hiy[i] = node.hiz[i] = -1e30f;
-            node.entry[i] = EMPTY_ENTRY;
-        }
-        float lo[3], hi[3];
-        padded(root.box, mag, lo, hi);
-        node.lox[0] = lo[0];
-        node.loy[0] = lo[1];
-        node.loz[0] = lo[2];
-        node.hix[0] = hi[0];
-        node.hiy[0] = hi[1];
-        node.hiz[0] = hi[2];
-        node.entry[0] = leaf_entry(root.first, root.count);
-        out.nodes.push_back(node);
-        out.depth = 1;
-        return out;
-    }
-    out.nodes.reserve(bld.next.load() / 2 + 2);
-    Collapser col{bld.nodes, out, mag};
-    col.collapse(0, 1);
-    return out;
-}
-
-BVH8 build_bvh8(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n,
-                int threads, int max_leaf, float traversal_cost) {
+// Binned-SAH tree over the finite triangles, collapsed into `Tree`.
+template <class Tree>
+Tree build_tree(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n, int threads,
+                int max_leaf, float traversal_cost) {
+    using Node = typename decltype(Tree::nodes)::value_type;
     if (threads <= 0) threads = int(std::max(1u, std::thread::hardware_concurrency()));
     Prepared pr = prepare(v0, e1, e2, n);
     const float mag = pr.mag;
     const uint32_t m = uint32_t(pr.order.size());
     Builder bld(pr.prims, std::move(pr.order), threads);
-    bld.max_leaf = uint32_t(std::min(std::max(max_leaf, 1), std::min(MAX_LEAF, BVH8_MAX_LEAF)));
+    bld.max_leaf = uint32_t(std::max(max_leaf, 1));
     bld.traversal_cost = traversal_cost > 0.f ? traversal_cost : 1.0f;
-    BVH8 out;
-    if (m == 0) {
-        BVH8Node node;
+    Tree out;
+    out.nodes.emplace_back();
+    if (m == 0) { // one node whose slots are all empty
+        Node& node = out.nodes[0];
         std::memset(&node, 0, sizeof(node));
-        std::memset(node.code, BVH8_EMPTY, 8);
-        std::memset(node.qlox, 255, 8);
-        std::memset(node.qloy, 255, 8);
-        std::memset(node.qloz, 255, 8);
-        node.ex = node.ey = node.ez = 0;
-        out.nodes.push_back(node);
+        std::memset(node.code, BVH8_EMPTY, sizeof(node.code));
+        for (uint8_t* q : {node.qlox, node.qloy, node.qloz}) std::memset(q, 255, sizeof(node.code));
         out.depth = 1;
+        out.max_exp = 0;
         return out;
     }
     bld.build(0, 0, m, 0);
-    out.nodes.reserve(bld.next.load() / 4 + 2);
+    out.nodes.reserve(bld.next.load() / 2 + 2);
     out.tris.reserve(m);
-    out.nodes.emplace_back();
-    Collapser8 col{bld.nodes, bld.idx, v0, e1, e2, flags, out, mag};
+    Collapser<Tree> col{bld.nodes, bld.idx, v0, e1, e2, flags, out, mag};
     col.emit(0, 0, 1);
     return out;
+}
+
+} // namespace
+
+BVH4 build_bvh4(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n,
+                int threads, int max_leaf, float traversal_cost) {
+    return build_tree<BVH4>(v0, e1, e2, flags, n, threads, std::min(max_leaf, MAX_LEAF), traversal_cost);
+}
+
+BVH8 build_bvh8(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n,
+                int threads, int max_leaf, float traversal_cost) {
+    return build_tree<BVH8>(v0, e1, e2, flags, n, threads, std::min(max_leaf, BVH8_MAX_LEAF), traversal_cost);
 }
 
 } // namespace mrt

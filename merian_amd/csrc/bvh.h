@@ -1,4 +1,4 @@
-// 4-wide BVH for the gfx950 traversal kernels: layout and host builder.
+// 4- and 8-wide quantised BVHs for the gfx950 traversal kernels: layouts and host builder.
 //
 // Replaces the driver acceleration-structure build of the reference
 // (src/merian/vk/raytrace/as_builder_blas.cpp:137, as_builder_tlas.cpp:131). Hit results do not
@@ -12,16 +12,6 @@
 
 namespace mrt {
 
-// One node = one 128-byte line: child boxes as structure-of-arrays so a lane reads them with
-// six 16-byte loads (lo/hi of one axis 16 bytes apart, so the ray's direction octant picks
-// the near and far plane by load address), then the four children as ready traversal entries.
-struct alignas(128) BVH4Node {
-    float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];
-    uint32_t entry[4];  // inner child: node index; leaf child: leaf entry (below); empty: 0xFFFFFFFF
-    uint32_t _pad[4];
-};
-static_assert(sizeof(BVH4Node) == 128, "BVH4Node must be one 128-byte line");
-
 // Triangle record in leaf order: the Moller-Trumbore operands, three 16-byte loads.
 //   a = (v0.xyz, id bits)   b = (e1.xyz, flags bits)   c = (e2.xyz, 0)
 // flags: bit 0 = back-face culling on, bits 8..15 = 8-bit instance mask.
@@ -31,16 +21,8 @@ struct alignas(16) TriRecord {
 
 // Leaf stack entries: bit 31 set, first record in bits 3..30, (count - 1) in bits 0..2.
 constexpr uint32_t LEAF_FLAG = 0x80000000u;
-constexpr uint32_t EMPTY_ENTRY = 0xFFFFFFFFu;
 inline uint32_t leaf_entry(uint32_t first, uint32_t count) { return LEAF_FLAG | (first << 3) | (count - 1u); }
 constexpr int MAX_LEAF = 8; // most triangles per leaf the encoding allows (the build default is 4)
-
-struct BVH4 {
-    std::vector<BVH4Node> nodes;   // nodes[0] is the root
-    std::vector<TriRecord> tris;   // leaf order
-    uint32_t depth = 0;            // longest root-to-leaf path in nodes
-    uint32_t root_leaf = 0;        // nonzero: the whole scene is one leaf entry (tiny scenes)
-};
 
 // v0/e1/e2: per-triangle float[3] operands exactly as the intersection test uses them
 // (e1 = v1 - v0, e2 = v2 - v0 rounded in float). flags as in TriRecord.
@@ -68,11 +50,45 @@ struct alignas(16) BVH8Node {
 static_assert(sizeof(BVH8Node) == 80, "BVH8Node must be 80 bytes");
 static_assert(BVH8_LEAF_CODE_MAX < BVH8_EMPTY, "leaf codes below the sentinels");
 
+// The same node for four children, 48 bytes: three 16-byte loads per visit (a traversal's loads are
+// scattered, one L1 access per lane and load, and the L1's address path is as busy as the vector
+// units: full-precision boxes cost seven loads). The grid exponent of an axis is the low byte of its
+// origin, whose float keeps 24 bits (rounded down).
+constexpr uint32_t BVH4_ORIGIN_MASK = 0xFFFFFF00u;
+struct alignas(16) BVH4Node {
+    uint32_t px, py, pz;    // grid origin (high 24 bits of the float) | exponent (int8) per axis
+    uint32_t child_base;
+    uint32_t tri_base;
+    uint8_t code[4];        // as BVH8Node.code
+    uint8_t qlox[4], qhix[4], qloy[4], qhiy[4], qloz[4], qhiz[4]; // empty slot: lo 255, hi 0
+};
+static_assert(sizeof(BVH4Node) == 48, "BVH4Node must be 48 bytes");
+static_assert(((3 * MAX_LEAF) << 3 | (MAX_LEAF - 1)) < BVH8_EMPTY, "leaf codes below the sentinels");
+
+// Null triangle records a device copy of `tris` ends with: the traversal may read an empty slot as a
+// leaf of one record, (BVH8_EMPTY >> 3) past a node's tri_base (mrt_trace.h).
+constexpr uint32_t TRI_PADDING = (BVH8_EMPTY >> 3) + 1u;
+
+struct BVH4 {
+    std::vector<BVH4Node> nodes; // nodes[0] is the root
+    std::vector<TriRecord> tris; // per node, its leaf children's triangles in slot order
+    uint32_t depth = 0;          // longest root-to-leaf path in nodes
+    int max_exp = -126;          // largest grid exponent
+};
+
 struct BVH8 {
     std::vector<BVH8Node> nodes; // nodes[0] is the root
     std::vector<TriRecord> tris; // per node, its leaf children's triangles in slot order
     uint32_t depth = 0;
+    int max_exp = -126;
 };
+
+// Smallest magnitude a direction component d takes in the box tests: 1e-20, and so large that
+// 2^(max_exp + 24) / d, the scale of the slab tests, stays finite (scenes beyond 2^45 units only).
+inline float bvh_dir_min(int max_exp) {
+    const int e = max_exp + 24 - 127;
+    return e > -66 ? __builtin_ldexpf(1.0f, e < 126 ? e : 126) : 1e-20f;
+}
 
 // max_leaf: most triangles per leaf (1..MAX_LEAF); traversal_cost: SAH cost of one node
 // visit relative to one triangle test.

@@ -194,8 +194,18 @@ __device__ __forceinline__ void flush_counts(const TraversalCount& c, unsigned l
 // ANY: visibility queries (first hit ends the traversal).
 // W: traversal of the scene's tree (4: BVH4Node; 8: quantised BVH8Node, sorted entries; 9: the
 // same nodes in octant order with grouped stack entries).
+// Waves per SIMD asked of the compiler (1: no limit on registers). A path queue's BVH8 traversal fits
+// 80 registers, six waves (the 1080p frame takes 169.0 ms, 171.3 with five). Camera rays hold more
+// per ray and a wave's rays end together: the 1080p GBuffer pass takes 505 us at the four waves its
+// registers allow, 550 with five, 573 with six. A ray array's BVH4 traversal fits 72 registers, seven
+// waves (4096x4096 camera rays 10.85 ms, 11.05 with six).
+template <class Src, int W> constexpr int TRACE_WAVES = W == 9 ? 5 : 1;
+template <> constexpr int TRACE_WAVES<SrcQueue, 8> = 6;
+template <> constexpr int TRACE_WAVES<SrcShadow, 8> = 6;
+template <> constexpr int TRACE_WAVES<SrcRays, 8> = 5;
+template <> constexpr int TRACE_WAVES<SrcRays, 4> = 7;
 template <bool COUNT, class Src, class Sink, bool ANY = false, int W = 4>
-__global__ __launch_bounds__(TRACE_BLOCK) void k_trace(DeviceScene S, Src src, Sink sink,
+__global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(TRACE_WAVES<Src, W>))) void k_trace(DeviceScene S, Src src, Sink sink,
                                                        const uint32_t* __restrict__ count_ptr, uint32_t n_fixed,
                                                        uint32_t* __restrict__ work, uint32_t mask, TraceScratch ts,
                                                        unsigned long long* counters) {
@@ -204,15 +214,15 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_trace(DeviceScene S, Src src, S
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const LaneStack stk{stack + threadIdx.x, ts.ovf + gtid, gridDim.x * blockDim.x};
     TraversalCount cnt;
+    auto run = [&](const auto bvh) {
+        trace_persistent<COUNT, ANY>(bvh, src, sink, n, work, mask, stk, cnt, ts.refill, ts.leaf_lanes, S.dir_min);
+    };
     if constexpr (W == 9) {
-        trace_persistent<TRACE_LDS_STACK, COUNT, Src, Sink, ANY>(DeviceBVH8G{S.nodes8, S.tris}, src, sink, n, work,
-                                                                 mask, stk, cnt, ts.refill, ts.leaf_lanes);
+        run(DeviceBVH8G{S.nodes8, S.tris});
     } else if constexpr (W == 8) {
-        trace_persistent<TRACE_LDS_STACK, COUNT, Src, Sink, ANY>(DeviceBVH8{S.nodes8, S.tris}, src, sink, n, work,
-                                                                 mask, stk, cnt, ts.refill, ts.leaf_lanes);
+        run(DeviceBVH8{S.nodes8, S.tris});
     } else {
-        trace_persistent<TRACE_LDS_STACK, COUNT, Src, Sink, ANY>(DeviceBVH{S.nodes, S.tris}, src, sink, n, work, mask,
-                                                                 stk, cnt, ts.refill, ts.leaf_lanes);
+        run(DeviceBVH4{S.nodes, S.tris});
     }
     if constexpr (COUNT) flush_counts(cnt, counters);
 }

@@ -34,6 +34,7 @@ struct DeviceScene {
     uint32_t n_tris;
     uint32_t n_geoms;
     uint32_t layered;            // some material has a coat or sheen lobe (material_layered)
+    float dir_min;               // smallest magnitude of a direction component in the box tests (bvh_dir_min)
     uint32_t stack_need;         // traversal stack entries the tree can need (width - 1 per level + slack)
 };
 
@@ -52,6 +53,10 @@ constexpr uint32_t TRI_SHADE_CLASS_SHIFT = 24;
 
 // Entries of the per-lane traversal stack kept in LDS; deeper entries go to TraceScratch.ovf.
 constexpr int TRACE_LDS_STACK = 16;
+// Overflow entries per lane for a stack of `need` entries.
+inline uint32_t trace_ovf_entries(uint32_t need) {
+    return need > uint32_t(TRACE_LDS_STACK) ? need - uint32_t(TRACE_LDS_STACK) : 1u;
+}
 // Threads per block of the trace kernels (also the LDS stack's column stride).
 constexpr int TRACE_BLOCK = 128;
 

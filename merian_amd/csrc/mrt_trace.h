@@ -1,6 +1,7 @@
-// Closest-hit traversal of the BVH4 (bvh.h) on gfx950: one ray per lane, the traversal stack
-// in LDS (one column per lane, so the 64 lanes of a wave hit 64 distinct banks), child order
-// near-to-far by a 4-key sorting network, octant-selected slab planes (one FMA per plane).
+// Closest-hit traversal of the quantised BVH4 and BVH8 (bvh.h) on gfx950: one ray per lane, the
+// traversal stack in LDS (one column per lane, so the 64 lanes of a wave hit distinct banks),
+// children near-to-far by a sort of integer keys, octant-selected slab planes (one byte permute
+// per two planes, one mixed-precision FMA per plane).
 //
 // Result = Scene.trace_ray (include/merian-shaders/scene/scene.slang:62-76) with the ray query
 // of acceleration-structure.slang:59-72: back-face culling per triangle, 8-bit instance mask,
@@ -16,11 +17,6 @@ namespace mrt {
 struct HitRec {
     uint32_t id; // global triangle id, 0xFFFFFFFF = miss
     float t, u, v;
-};
-
-struct DeviceBVH {
-    const BVH4Node* nodes;
-    const float4* tris; // TriRecord as 3 x float4
 };
 
 // Textbook Moller-Trumbore (1997) in a fixed operation order; no contraction (the file is
@@ -50,61 +46,38 @@ __device__ __forceinline__ void test_triangle(const float4 A, const float4 B, co
     if (t < best.t || (t == best.t && id < best.id)) best = HitRec{id, t, u, v};
 }
 
-__device__ __forceinline__ void cswap(float& ka, uint32_t& ea, float& kb, uint32_t& eb) {
-    const bool s = kb < ka;
-    const float tk = s ? kb : ka;
-    const uint32_t te = s ? eb : ea;
-    kb = s ? ka : kb;
-    eb = s ? ea : eb;
-    ka = tk;
-    ea = te;
-}
-
 constexpr uint32_t TRAVERSAL_DONE = 0xFFFFFFFFu;
+constexpr int KEY_MISS = 0x7FFFFFFF; // sort key of a child whose box is missed: above every limit
 
 // Work counters of one traversal (COUNT variant only): node visits and triangle tests.
 struct TraversalCount {
     uint32_t nodes = 0, tris = 0;
 };
 
-// Traversal stack of one lane: the first SL entries in an LDS column (stride = threads per
-// block, so a wave's 64 lanes touch 64 distinct banks), deeper entries in a per-lane column of a
-// global overflow area (stride = threads of the grid). Near-first traversal rarely goes past SL.
-// The LDS column stride is the block size, a compile-time constant (a shift, not a multiply).
+// Traversal stack of one lane: the first TRACE_LDS_STACK entries in an LDS column (stride = threads
+// per block, a compile-time constant, so a wave's 64 lanes touch 64 distinct banks), deeper entries
+// in a per-lane column of a global overflow area (stride = threads of the grid). Near-first
+// traversal rarely goes past the LDS part.
+typedef __attribute__((address_space(3))) uint32_t* lds_u32;
+typedef __attribute__((address_space(1))) uint32_t* global_u32;
 struct LaneStack {
     uint32_t* lds; // this lane's column
     uint32_t* ovf;
     uint32_t ovf_stride;
 };
-template <int SL> __device__ __forceinline__ void stack_push(const LaneStack& s, int& sp, uint32_t e) {
-    if (sp < SL) {
-        s.lds[sp * TRACE_BLOCK] = e;
+// explicit address spaces keep LDS and overflow accesses apart (ds and global instructions rather
+// than flat ones through a selected pointer)
+__device__ __forceinline__ void stack_poke(const LaneStack& s, int i, uint32_t e) {
+    if (i < TRACE_LDS_STACK) {
+        ((lds_u32)s.lds)[i * TRACE_BLOCK] = e;
     } else {
-        s.ovf[size_t(sp - SL) * s.ovf_stride] = e;
+        ((global_u32)s.ovf)[size_t(i - TRACE_LDS_STACK) * s.ovf_stride] = e;
     }
-    sp++;
 }
-template <int SL> __device__ __forceinline__ uint32_t stack_pop(const LaneStack& s, int& sp) {
-    --sp;
-    // explicit address spaces keep the two loads apart (a ds_read and a global load rather
-    // than one flat load through a selected pointer)
-    typedef const __attribute__((address_space(3))) uint32_t* lds_ptr;
-    typedef const __attribute__((address_space(1))) uint32_t* global_ptr;
-    if (sp < SL) return ((lds_ptr)s.lds)[sp * TRACE_BLOCK];
-    return ((global_ptr)s.ovf)[size_t(sp - SL) * s.ovf_stride];
-}
-template <int SL> __device__ __forceinline__ uint32_t stack_peek(const LaneStack& s, int i) {
-    typedef const __attribute__((address_space(3))) uint32_t* lds_ptr;
-    typedef const __attribute__((address_space(1))) uint32_t* global_ptr;
-    if (i < SL) return ((lds_ptr)s.lds)[i * TRACE_BLOCK];
-    return ((global_ptr)s.ovf)[size_t(i - SL) * s.ovf_stride];
-}
-template <int SL> __device__ __forceinline__ void stack_poke(const LaneStack& s, int i, uint32_t e) {
-    if (i < SL) {
-        s.lds[i * TRACE_BLOCK] = e;
-    } else {
-        s.ovf[size_t(i - SL) * s.ovf_stride] = e;
-    }
+__device__ __forceinline__ void stack_push(const LaneStack& s, int& sp, uint32_t e) { stack_poke(s, sp++, e); }
+__device__ __forceinline__ uint32_t stack_peek(const LaneStack& s, int i) {
+    if (i < TRACE_LDS_STACK) return ((lds_u32)s.lds)[i * TRACE_BLOCK];
+    return ((global_u32)s.ovf)[size_t(i - TRACE_LDS_STACK) * s.ovf_stride];
 }
 
 // Per-lane traversal state between steps.
@@ -112,12 +85,11 @@ struct RayState {
     f3 o, d;
     float ix, iy, iz, ox, oy, oz;
     float t0, tmin, tmax;
-    float tlim;   // far limit of the box tests: min(tmax, best.t) widened by 2 ulp
+    int klim;     // far limit of the box tests as a sort key (key_limit)
     uint32_t neg; // bit k: direction component k is negative
-    uint32_t pn, pf; // BVH4: byte offsets of the near / far plane row of axis k in byte k
-    uint32_t psel[3]; // BVH8: v_perm selector per axis picking the near plane word of a node
-                      // (lo for a positive direction, hi for a negative one); swapped operands
-                      // pick the far word
+    uint32_t psel[3]; // v_perm selector per axis: the near planes of children 0 and 1 (lo for a
+                      // positive direction, hi for a negative one) as two zero-extended bytes;
+                      // + 0x00020002: children 2 and 3; swapped operands: the far planes
     HitRec best;
     int sp;
     uint32_t cur;  // next entry to process; TRAVERSAL_DONE when the stack is exhausted
@@ -127,12 +99,23 @@ struct RayState {
 __device__ __forceinline__ bool is_inner(uint32_t e) { return !(e & LEAF_FLAG); }
 __device__ __forceinline__ bool is_leaf(uint32_t e) { return e != TRAVERSAL_DONE && (e & LEAF_FLAG); }
 
-__device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, float tmax) {
+// Far limit of the box tests, min(tmax, best.t) widened by 2 ulp, as a sort key: a child is
+// visited while its key is at most this. Keys compare as signed integers, so non-negative
+// distances compare as they should and a negative one (a box around the origin of a ray with a
+// negative tmin) is below every limit; a negative limit (nothing can be hit) admits everything
+// and leaves the rejection to the triangle test.
+__device__ __forceinline__ int key_limit(float tmax, float t) {
+    const float lim = fminf(tmax, t) * 1.00000024f;
+    return lim >= 0.f ? int(__float_as_uint(fabsf(lim)) | 0xFFu) : KEY_MISS - 1; // fabsf: -0 is 0
+}
+
+// dir_min: smallest magnitude of a direction component in the box tests (DeviceScene.dir_min).
+__device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, float tmax, float dir_min) {
     r.o = o;
     r.d = d;
-    const float dx = fabsf(d.x) < 1e-20f ? copysignf(1e-20f, d.x) : d.x;
-    const float dy = fabsf(d.y) < 1e-20f ? copysignf(1e-20f, d.y) : d.y;
-    const float dz = fabsf(d.z) < 1e-20f ? copysignf(1e-20f, d.z) : d.z;
+    const float dx = fabsf(d.x) < dir_min ? copysignf(dir_min, d.x) : d.x;
+    const float dy = fabsf(d.y) < dir_min ? copysignf(dir_min, d.y) : d.y;
+    const float dz = fabsf(d.z) < dir_min ? copysignf(dir_min, d.z) : d.z;
     // the hardware reciprocal (1 ulp) instead of a correctly rounded division: 1/d only feeds
     // the box tests, whose boxes the builder pads by extent/1024 + magnitude/65536, far above
     // an ulp of the slab distances; the triangle test uses d itself
@@ -147,21 +130,17 @@ __device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, f
     r.tmax = tmax;
     r.t0 = tmin - fabsf(tmin) * 2.4e-7f;
     r.best = HitRec{TRAVERSAL_DONE, __builtin_inff(), 0.f, 0.f};
-    r.tlim = fminf(tmax, r.best.t) * 1.00000024f;
-    // BVH4Node rows: lox hix loy hiy loz hiz, 16 bytes each
-    const uint32_t nx = r.neg & 1u, ny = (r.neg >> 1) & 1u, nz = (r.neg >> 2) & 1u;
-    r.pn = (nx << 4) | ((32u + (ny << 4)) << 8) | ((64u + (nz << 4)) << 16);
-    r.pf = ((16u - (nx << 4))) | ((48u - (ny << 4)) << 8) | ((80u - (nz << 4)) << 16);
-    r.psel[0] = nx ? 0x07060504u : 0x03020100u;
-    r.psel[1] = ny ? 0x07060504u : 0x03020100u;
-    r.psel[2] = nz ? 0x07060504u : 0x03020100u;
+    r.klim = key_limit(tmax, r.best.t);
+    r.psel[0] = (r.neg & 1u) ? 0x0C050C04u : 0x0C010C00u;
+    r.psel[1] = (r.neg & 2u) ? 0x0C050C04u : 0x0C010C00u;
+    r.psel[2] = (r.neg & 4u) ? 0x0C050C04u : 0x0C010C00u;
     r.sp = 0;
     r.cur = 0u; // root node (always an inner node)
     r.leaf = TRAVERSAL_DONE;
 }
 
 // Tests the triangles of the postponed leaf (ANY: the first hit ends the traversal).
-template <int SL, bool COUNT, bool ANY>
+template <bool COUNT, bool ANY>
 __device__ __forceinline__ void leaf_test(const float4* __restrict__ tris, RayState& r, uint32_t ray_mask,
                                           TraversalCount& count) {
     const uint32_t first = (r.leaf & 0x7FFFFFFFu) >> 3;
@@ -176,7 +155,7 @@ __device__ __forceinline__ void leaf_test(const float4* __restrict__ tris, RaySt
     }
     if constexpr (COUNT) count.tris += cnt;
     r.leaf = TRAVERSAL_DONE;
-    r.tlim = fminf(r.tmax, r.best.t) * 1.00000024f;
+    r.klim = key_limit(r.tmax, r.best.t);
     if constexpr (ANY) {
         if (r.best.id != TRAVERSAL_DONE) {
             r.cur = TRAVERSAL_DONE;
@@ -185,246 +164,211 @@ __device__ __forceinline__ void leaf_test(const float4* __restrict__ tris, RaySt
     }
 }
 
-// One inner-node step (r.cur is an inner node): test its four children, push the hit ones far
-// to near, continue with the nearest.
-template <int SL, bool COUNT>
-__device__ __forceinline__ void node_step(const DeviceBVH bvh, RayState& r, const LaneStack& stk,
-                                          TraversalCount& count) {
-    if constexpr (COUNT) count.nodes++;
-    // near and far plane rows of each axis chosen by address: one FMA per plane, no selects
-    const char* nb = reinterpret_cast<const char*>(bvh.nodes);
-    const uint32_t off = r.cur << 7;
-    auto row = [&](uint32_t o) { return *reinterpret_cast<const float4*>(nb + (off + o)); };
-    const float4 nxr = row(r.pn & 0xFFu), fxr = row(r.pf & 0xFFu);
-    const float4 nyr = row((r.pn >> 8) & 0xFFu), fyr = row((r.pf >> 8) & 0xFFu);
-    const float4 nzr = row(r.pn >> 16), fzr = row(r.pf >> 16);
-    const uint4 ent4 = *reinterpret_cast<const uint4*>(nb + (off + 96u));
-    const float tlim = r.tlim;
-    float key[4];
-    uint32_t ent[4];
-#define MRT_CHILD(c, NX, FX, NY, FY, NZ, FZ, E)                                                              \
-    {                                                                                                        \
-        const float tn = fmaxf(fmaxf(__builtin_fmaf(NX, r.ix, -r.ox), __builtin_fmaf(NY, r.iy, -r.oy)),      \
-                               fmaxf(__builtin_fmaf(NZ, r.iz, -r.oz), r.t0));                               \
-        const float tf = fminf(fminf(__builtin_fmaf(FX, r.ix, -r.ox), __builtin_fmaf(FY, r.iy, -r.oy)),      \
-                               fminf(__builtin_fmaf(FZ, r.iz, -r.oz), tlim));                               \
-        key[c] = (tn <= tf) ? tn : __builtin_inff();                                                         \
-        ent[c] = E;                                                                                          \
-    }
-    MRT_CHILD(0, nxr.x, fxr.x, nyr.x, fyr.x, nzr.x, fzr.x, ent4.x)
-    MRT_CHILD(1, nxr.y, fxr.y, nyr.y, fyr.y, nzr.y, fzr.y, ent4.y)
-    MRT_CHILD(2, nxr.z, fxr.z, nyr.z, fyr.z, nzr.z, fzr.z, ent4.z)
-    MRT_CHILD(3, nxr.w, fxr.w, nyr.w, fyr.w, nzr.w, fzr.w, ent4.w)
-#undef MRT_CHILD
-    cswap(key[0], ent[0], key[1], ent[1]);
-    cswap(key[2], ent[2], key[3], ent[3]);
-    cswap(key[0], ent[0], key[2], ent[2]);
-    cswap(key[1], ent[1], key[3], ent[3]);
-    cswap(key[1], ent[1], key[2], ent[2]);
-    const float inf = __builtin_inff();
-    if (key[3] != inf) stack_push<SL>(stk, r.sp, ent[3]);
-    if (key[2] != inf) stack_push<SL>(stk, r.sp, ent[2]);
-    if (key[1] != inf) stack_push<SL>(stk, r.sp, ent[1]);
-    if (key[0] != inf) {
-        r.cur = ent[0];
-    } else {
-        r.cur = r.sp > 0 ? stack_pop<SL>(stk, r.sp) : TRAVERSAL_DONE;
-    }
-}
-
-// Entry of BVH8 slot c from the node's second 16 bytes (child base, triangle base, code words):
-// the slot's code byte picked by a byte permute (selector bytes 0x0C read as zero), then
-// base + code (bvh.h).
-__device__ __forceinline__ uint32_t bvh8_entry(const uint4 h1, uint32_t c) {
-    const uint32_t code = __builtin_amdgcn_perm(h1.w, h1.z, c | 0x0C0C0C00u);
-    return (code >= BVH8_INNER ? h1.x - uint32_t(BVH8_INNER) : LEAF_FLAG | (h1.y << 3)) + code;
+// Entry of a slot from its node's child base and triangle base and its code byte (bvh.h).
+__device__ __forceinline__ uint32_t code_entry(uint32_t child_base, uint32_t tri_base, uint32_t code) {
+    return (code >= BVH8_INNER ? child_base - uint32_t(BVH8_INNER) : LEAF_FLAG | (tri_base << 3)) + code;
 }
 
 // Grouped BVH8 stack entries: a node index (< 2^24) and, in the top byte, the node's hit
 // children not yet visited as a mask over visiting positions (position i = slot i ^ r.neg).
 constexpr uint32_t BVH8_GROUP_NODE = 0xFFFFFFu;
 
-struct DeviceBVH8 { // near-first order by sorted distances, one stack entry per pushed child
-    const BVH8Node* nodes;
+// The trees as the traversal reads them. W: children per node.
+struct DeviceBVH4 { // near-first order by sorted distances, one stack entry per pushed child
+    static constexpr int W = 4;
+    static constexpr bool SORTED = true;
+    const BVH4Node* nodes;
     const float4* tris; // TriRecord as 3 x float4
 };
+struct DeviceBVH8 {
+    static constexpr int W = 8;
+    static constexpr bool SORTED = true;
+    const BVH8Node* nodes;
+    const float4* tris;
+};
 struct DeviceBVH8G { // octant visiting order, one stack group per node
+    static constexpr int W = 8;
+    static constexpr bool SORTED = false;
     const BVH8Node* nodes;
     const float4* tris;
 };
 
-// Next entry to visit: BVH4 and sorted BVH8 pop a ready entry; grouped BVH8 takes the first
-// remaining child of the top group (re-reading its node's 16-byte header) and drops the group
-// once it is empty.
-template <int SL>
-__device__ __forceinline__ uint32_t pop_next(const DeviceBVH&, RayState& r, const LaneStack& stk) {
-    return r.sp > 0 ? stack_pop<SL>(stk, r.sp) : TRAVERSAL_DONE;
-}
-template <int SL>
-__device__ __forceinline__ uint32_t pop_next(const DeviceBVH8&, RayState& r, const LaneStack& stk) {
-    return r.sp > 0 ? stack_pop<SL>(stk, r.sp) : TRAVERSAL_DONE;
-}
-template <int SL>
-__device__ __forceinline__ uint32_t pop_next(const DeviceBVH8G bvh, RayState& r, const LaneStack& stk) {
+// Next entry to visit: sorted trees pop a ready entry; grouped BVH8 takes the first remaining child
+// of the top group (re-reading its node's 16-byte header) and drops the group once it is empty.
+template <class BVH> __device__ __forceinline__ uint32_t pop_next(const BVH bvh, RayState& r, const LaneStack& stk) {
     if (r.sp == 0) return TRAVERSAL_DONE;
-    const uint32_t g = stack_peek<SL>(stk, r.sp - 1);
-    const uint32_t node = g & BVH8_GROUP_NODE;
-    const uint32_t m = g >> 24;
-    const uint4 h1 = reinterpret_cast<const uint4*>(bvh.nodes + node)[1];
-    const uint32_t rest = m & (m - 1u);
-    if (rest == 0u) {
-        r.sp--;
+    if constexpr (BVH::SORTED) {
+        return stack_peek(stk, --r.sp);
     } else {
-        stack_poke<SL>(stk, r.sp - 1, node | (rest << 24));
+        const uint32_t g = stack_peek(stk, r.sp - 1);
+        const uint32_t node = g & BVH8_GROUP_NODE;
+        const uint32_t m = g >> 24;
+        const uint4 h1 = reinterpret_cast<const uint4*>(bvh.nodes + node)[1];
+        const uint32_t rest = m & (m - 1u);
+        if (rest == 0u) {
+            r.sp--;
+        } else {
+            stack_poke(stk, r.sp - 1, node | (rest << 24));
+        }
+        const uint32_t c = uint32_t(__builtin_ctz(m)) ^ r.neg;
+        return code_entry(h1.x, h1.y, __builtin_amdgcn_perm(h1.w, h1.z, c | 0x0C0C0C00u));
     }
-    return bvh8_entry(h1, uint32_t(__builtin_ctz(m)) ^ r.neg);
 }
 
-// One inner-node step over the 8-wide quantised BVH, near-first by sorted entry distance: slab-test the eight child boxes, sort the
-// hit children near to far, push all but the nearest, continue with it.
+// A node as read: grid origin and steps, bases, codes, and per axis the lo / hi plane bytes of
+// children 0-3 and (W = 8) 4-7.
+template <int W> struct NodeData {
+    float px, py, pz;
+    int ex, ey, ez;
+    uint32_t child_base, tri_base, code[W / 4];
+    uint32_t lo[3][W / 4], hi[3][W / 4];
+};
+__device__ __forceinline__ NodeData<8> load_node(const BVH8Node* n) {
+    const uint4* p = reinterpret_cast<const uint4*>(n);
+    const uint4 h0 = p[0], h1 = p[1], qx = p[2], qy = p[3], qz = p[4];
+    return NodeData<8>{__uint_as_float(h0.x), __uint_as_float(h0.y), __uint_as_float(h0.z),
+                       int(int8_t(h0.w & 0xFFu)), int(int8_t((h0.w >> 8) & 0xFFu)), int(int8_t((h0.w >> 16) & 0xFFu)),
+                       h1.x, h1.y, {h1.z, h1.w},
+                       {{qx.x, qx.y}, {qy.x, qy.y}, {qz.x, qz.y}}, {{qx.z, qx.w}, {qy.z, qy.w}, {qz.z, qz.w}}};
+}
+__device__ __forceinline__ NodeData<4> load_node(const BVH4Node* n) {
+    const uint4* p = reinterpret_cast<const uint4*>(n);
+    const uint4 h0 = p[0], h1 = p[1], h2 = p[2];
+    return NodeData<4>{__uint_as_float(h0.x & BVH4_ORIGIN_MASK), __uint_as_float(h0.y & BVH4_ORIGIN_MASK),
+                       __uint_as_float(h0.z & BVH4_ORIGIN_MASK), int(int8_t(h0.x & 0xFFu)), int(int8_t(h0.y & 0xFFu)),
+                       int(int8_t(h0.z & 0xFFu)), h0.w, h1.x, {h1.y}, {{h1.z}, {h2.x}, {h2.z}}, {{h1.w}, {h2.y}, {h2.w}}};
+}
+
+// Slab tests of the node's W child boxes: entry and exit distance per child (tn clamped to the
+// ray's near limit, tf not clamped to its far limit).
 //
-// Slab distances are taken in the node's grid: a plane at grid coordinate q lies at q 2^e + p,
-// so its distance is q (2^e / d) + (p / d - o / d) = fma(q, a, b) with a = 2^e ix (exact: a
-// power-of-two scale) and b = fma(p, ix, -ox) once per node and axis, one FMA per plane after
-// the byte conversion. The sort key of a hit child is its entry distance's bit pattern with the
-// child slot in the low three bits (misses: all ones), so a 19-comparator network of integer
-// min/max sorts keys alone; a pushed child's entry is rebuilt from its slot's code byte.
+// Distances are taken in the node's grid: a plane at grid coordinate q lies at q 2^e + p, so its
+// distance is q (2^e / d) + (p / d - o / d) = fma(q, a, b) with a = 2^e ix (exact: a power-of-two
+// scale) and b = fma(p, ix, -ox) once per node and axis. A plane's byte, zero-extended to 16
+// bits by the byte permute that picks near or far planes of two children at once, is the half
+// float q 2^-24 (a denormal, exact), which the mixed-precision FMA takes as its first operand; a
+// carries the factor 2^24. So a plane costs half a permute and an FMA, against half a permute of
+// four, a byte conversion and an FMA before (the same values: q a is rounded once, in the FMA).
+template <int W>
+__device__ __forceinline__ void slab_tests(const NodeData<W>& n, const RayState& r, float (&tn)[W], float (&tf)[W]) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const float a[3] = {ldexpf(r.ix, n.ex + 24), ldexpf(r.iy, n.ey + 24), ldexpf(r.iz, n.ez + 24)};
+    const float b[3] = {__builtin_fmaf(n.px, r.ix, -r.ox), __builtin_fmaf(n.py, r.iy, -r.oy),
+                        __builtin_fmaf(n.pz, r.iz, -r.oz)};
+#pragma unroll
+    for (int p = 0; p < W / 2; p++) { // children 2 p, 2 p + 1
+        const int w = p >> 1;
+        float nr[3][2], fr[3][2];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const uint32_t sel = r.psel[k] + ((p & 1) ? 0x00020002u : 0u);
+            const h2 qn = __builtin_bit_cast(h2, __builtin_amdgcn_perm(n.hi[k][w], n.lo[k][w], sel));
+            const h2 qf = __builtin_bit_cast(h2, __builtin_amdgcn_perm(n.lo[k][w], n.hi[k][w], sel));
+            nr[k][0] = __builtin_fmaf(float(qn.x), a[k], b[k]);
+            nr[k][1] = __builtin_fmaf(float(qn.y), a[k], b[k]);
+            fr[k][0] = __builtin_fmaf(float(qf.x), a[k], b[k]);
+            fr[k][1] = __builtin_fmaf(float(qf.y), a[k], b[k]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            tn[2 * p + j] = fmaxf(fmaxf(nr[0][j], nr[1][j]), fmaxf(nr[2][j], r.t0));
+            tf[2 * p + j] = fminf(fminf(fr[0][j], fr[1][j]), fr[2][j]);
+        }
+    }
+}
+
+__device__ __forceinline__ int med3(int a, int b, int c) { return max(min(a, b), min(max(a, b), c)); }
+
+// One inner-node step (r.cur is an inner node), near-first by sorted entry distance: sort the
+// children near to far, push the hit ones but the nearest, continue with the nearest.
+//
+// The sort key of a child is its entry distance's bit pattern with the slot's code byte in place of
+// the low byte (one byte permute; a missed box: KEY_MISS), so a key holds all that a pushed child's
+// entry needs. The far limit is applied to the sorted keys (key <= klim), not to every box. Keys are
+// sorted by insertion: a key d goes into a sorted list s by out[i] = med3(s[i - 1], s[i], d), one
+// instruction per element (33 for eight keys, 7 for four, against 38 and 10 of a compare-exchange
+// network).
+// An empty slot (an inverted box) can only pass if all its plane distances round to one value; it
+// then reads as a leaf of one record at most 30 past the node's own, which the triangle array's
+// padding keeps in bounds: one more triangle tested, or a null record. So slots are not checked
+// for being empty.
 // Only the visiting order depends on the keys; which children are visited does not.
-template <int SL, bool COUNT>
-__device__ __forceinline__ void node_step(const DeviceBVH8 bvh, RayState& r, const LaneStack& stk,
-                                          TraversalCount& count) {
+template <bool COUNT, class BVH>
+__device__ __forceinline__ void node_step(const BVH bvh, RayState& r, const LaneStack& stk, TraversalCount& count) {
+    constexpr int W = BVH::W;
     if constexpr (COUNT) count.nodes++;
-    const uint4* np = reinterpret_cast<const uint4*>(bvh.nodes + r.cur);
-    const uint4 h0 = np[0], h1 = np[1], qx = np[2], qy = np[3], qz = np[4];
-    const int ex = int(int8_t(h0.w & 0xFFu)), ey = int(int8_t((h0.w >> 8) & 0xFFu)), ez = int(int8_t((h0.w >> 16) & 0xFFu));
-    const float ax = ldexpf(r.ix, ex), ay = ldexpf(r.iy, ey), az = ldexpf(r.iz, ez); // 2^e ix, exact
-    const float bx = __builtin_fmaf(__uint_as_float(h0.x), r.ix, -r.ox);
-    const float by = __builtin_fmaf(__uint_as_float(h0.y), r.iy, -r.oy);
-    const float bz = __builtin_fmaf(__uint_as_float(h0.z), r.iz, -r.oz);
-    const float tlim = r.tlim;
-    // near / far plane bytes per axis, picked by the ray's octant with one byte permute per word
-    // (children 0-3 in the low word, 4-7 in the high word)
-    const uint32_t sx = r.psel[0], sy = r.psel[1], sz = r.psel[2];
-    const uint32_t nx0 = __builtin_amdgcn_perm(qx.z, qx.x, sx), nx1 = __builtin_amdgcn_perm(qx.w, qx.y, sx);
-    const uint32_t fx0 = __builtin_amdgcn_perm(qx.x, qx.z, sx), fx1 = __builtin_amdgcn_perm(qx.y, qx.w, sx);
-    const uint32_t ny0 = __builtin_amdgcn_perm(qy.z, qy.x, sy), ny1 = __builtin_amdgcn_perm(qy.w, qy.y, sy);
-    const uint32_t fy0 = __builtin_amdgcn_perm(qy.x, qy.z, sy), fy1 = __builtin_amdgcn_perm(qy.y, qy.w, sy);
-    const uint32_t nz0 = __builtin_amdgcn_perm(qz.z, qz.x, sz), nz1 = __builtin_amdgcn_perm(qz.w, qz.y, sz);
-    const uint32_t fz0 = __builtin_amdgcn_perm(qz.x, qz.z, sz), fz1 = __builtin_amdgcn_perm(qz.y, qz.w, sz);
-    constexpr uint32_t MISS = 0xFFFFFFFFu;
-    uint32_t key[8];
+    const NodeData<W> n = load_node(bvh.nodes + r.cur);
+    float tn[W], tf[W];
+    slab_tests(n, r, tn, tf);
+    if constexpr (BVH::SORTED) {
+        int key[W];
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint32_t sh = 8u * uint32_t(c & 3);
-        const float NX = __builtin_fmaf(float(((c < 4 ? nx0 : nx1) >> sh) & 0xFFu), ax, bx);
-        const float FX = __builtin_fmaf(float(((c < 4 ? fx0 : fx1) >> sh) & 0xFFu), ax, bx);
-        const float NY = __builtin_fmaf(float(((c < 4 ? ny0 : ny1) >> sh) & 0xFFu), ay, by);
-        const float FY = __builtin_fmaf(float(((c < 4 ? fy0 : fy1) >> sh) & 0xFFu), ay, by);
-        const float NZ = __builtin_fmaf(float(((c < 4 ? nz0 : nz1) >> sh) & 0xFFu), az, bz);
-        const float FZ = __builtin_fmaf(float(((c < 4 ? fz0 : fz1) >> sh) & 0xFFu), az, bz);
-        const float tn = fmaxf(fmaxf(NX, NY), fmaxf(NZ, r.t0));
-        const float tf = fminf(fminf(FX, FY), fminf(FZ, tlim));
-        const uint32_t code = ((c < 4 ? h1.z : h1.w) >> sh) & 0xFFu;
-        key[c] = (tn <= tf && code != BVH8_EMPTY) ? ((__float_as_uint(tn) & ~7u) | uint32_t(c)) : MISS;
-    }
-    // entry of the slot in a sorted key's low bits
-    auto entry_of = [&](uint32_t k) { return bvh8_entry(h1, k & 7u); };
-#define MRT_CS(a, b)                                                                                           \
-    {                                                                                                          \
-        const uint32_t lo_ = min(key[a], key[b]);                                                              \
-        key[b] = max(key[a], key[b]);                                                                          \
-        key[a] = lo_;                                                                                          \
-    }
-    MRT_CS(0, 1) MRT_CS(2, 3) MRT_CS(4, 5) MRT_CS(6, 7)
-    MRT_CS(0, 2) MRT_CS(1, 3) MRT_CS(4, 6) MRT_CS(5, 7)
-    MRT_CS(1, 2) MRT_CS(5, 6)
-    MRT_CS(0, 4) MRT_CS(1, 5) MRT_CS(2, 6) MRT_CS(3, 7)
-    MRT_CS(2, 4) MRT_CS(3, 5)
-    MRT_CS(1, 2) MRT_CS(3, 4) MRT_CS(5, 6)
-#undef MRT_CS
+        for (int c = 0; c < W; c++) {
+            const uint32_t k = __builtin_amdgcn_perm(__float_as_uint(tn[c]), n.code[c >> 2], 0x07060500u | uint32_t(c & 3));
+            const int d = tn[c] <= tf[c] ? int(k) : KEY_MISS;
+            // key[0 .. c - 1] is sorted: insert d
+            int prev = d;
 #pragma unroll
-    for (int c = 7; c >= 1; c--)
-        if (key[c] != MISS) stack_push<SL>(stk, r.sp, entry_of(key[c]));
-    if (key[0] != MISS) {
-        r.cur = entry_of(key[0]);
+            for (int i = 0; i < c; i++) {
+                const int s = key[i];
+                key[i] = i == 0 ? min(s, d) : med3(prev, s, d);
+                prev = s;
+            }
+            key[c] = c == 0 ? d : max(prev, d);
+        }
+        const uint32_t inner_base = n.child_base - uint32_t(BVH8_INNER), leaf_base = LEAF_FLAG | (n.tri_base << 3);
+        auto entry_of = [&](int k) {
+            const uint32_t code = uint32_t(k) & 0xFFu;
+            return (code >= BVH8_INNER ? inner_base : leaf_base) + code;
+        };
+        // far to near; the whole wave writes to LDS unless a lane's stack may leave it
+        if (__any(r.sp > TRACE_LDS_STACK - (W - 1))) {
+#pragma unroll
+            for (int c = W - 1; c >= 1; c--)
+                if (key[c] <= r.klim) stack_push(stk, r.sp, entry_of(key[c]));
+        } else {
+#pragma unroll
+            for (int c = W - 1; c >= 1; c--)
+                if (key[c] <= r.klim) ((lds_u32)stk.lds)[r.sp++ * TRACE_BLOCK] = entry_of(key[c]);
+        }
+        r.cur = key[0] <= r.klim ? entry_of(key[0]) : pop_next(bvh, r, stk);
     } else {
-        r.cur = r.sp > 0 ? stack_pop<SL>(stk, r.sp) : TRAVERSAL_DONE;
-    }
-}
-
-
-// One inner-node step over the 8-wide quantised BVH in octant order: slab-test the eight child
-// boxes, continue with the first hit child in the ray's visiting order and push the others as
-// one group. Fewer instructions per node than the sorted step, but a pop re-reads a node
-// header: it wins on long incoherent traversals and loses where pops are frequent.
-//
-// Slab distances are taken in the node's grid: a plane at grid coordinate q lies at q 2^e + p,
-// so its distance is q (2^e / d) + (p / d - o / d) = fma(q, a, b) with a = 2^e ix (exact: a
-// power-of-two scale) and b = fma(p, ix, -ox) once per node and axis, one FMA per plane after
-// the byte conversion. Visiting order: the builder puts a child in the slot of the node corner
-// it lies toward (bit a: high end of axis a), so a ray whose direction signs are r.neg meets
-// them roughly in the order slot = i ^ r.neg, i = 0..7 (the ordering of compressed wide BVHs,
-// Ylitie, Karras and Laine 2017); the hit mask is permuted into that order by three
-// conditional bit-group swaps, and no distances are sorted. Only the visiting order depends on
-// it; which children are visited does not.
-template <int SL, bool COUNT>
-__device__ __forceinline__ void node_step(const DeviceBVH8G bvh, RayState& r, const LaneStack& stk,
-                                          TraversalCount& count) {
-    if constexpr (COUNT) count.nodes++;
-    const uint4* np = reinterpret_cast<const uint4*>(bvh.nodes + r.cur);
-    const uint4 h0 = np[0], h1 = np[1], qx = np[2], qy = np[3], qz = np[4];
-    const int ex = int(int8_t(h0.w & 0xFFu)), ey = int(int8_t((h0.w >> 8) & 0xFFu)), ez = int(int8_t((h0.w >> 16) & 0xFFu));
-    const float ax = ldexpf(r.ix, ex), ay = ldexpf(r.iy, ey), az = ldexpf(r.iz, ez); // 2^e ix, exact
-    const float bx = __builtin_fmaf(__uint_as_float(h0.x), r.ix, -r.ox);
-    const float by = __builtin_fmaf(__uint_as_float(h0.y), r.iy, -r.oy);
-    const float bz = __builtin_fmaf(__uint_as_float(h0.z), r.iz, -r.oz);
-    const float tlim = r.tlim;
-    // near / far plane bytes per axis, picked by the ray's octant with one byte permute per word
-    // (children 0-3 in the low word, 4-7 in the high word)
-    const uint32_t sx = r.psel[0], sy = r.psel[1], sz = r.psel[2];
-    const uint32_t nx0 = __builtin_amdgcn_perm(qx.z, qx.x, sx), nx1 = __builtin_amdgcn_perm(qx.w, qx.y, sx);
-    const uint32_t fx0 = __builtin_amdgcn_perm(qx.x, qx.z, sx), fx1 = __builtin_amdgcn_perm(qx.y, qx.w, sx);
-    const uint32_t ny0 = __builtin_amdgcn_perm(qy.z, qy.x, sy), ny1 = __builtin_amdgcn_perm(qy.w, qy.y, sy);
-    const uint32_t fy0 = __builtin_amdgcn_perm(qy.x, qy.z, sy), fy1 = __builtin_amdgcn_perm(qy.y, qy.w, sy);
-    const uint32_t nz0 = __builtin_amdgcn_perm(qz.z, qz.x, sz), nz1 = __builtin_amdgcn_perm(qz.w, qz.y, sz);
-    const uint32_t fz0 = __builtin_amdgcn_perm(qz.x, qz.z, sz), fz1 = __builtin_amdgcn_perm(qz.y, qz.w, sz);
-    uint32_t hm = 0u; // bit c: slot c is hit
+        // Octant order: continue with the first hit child in the ray's visiting order and push the
+        // others as one group. Fewer instructions per node than the sorted step, but a pop re-reads
+        // a node header: it wins on long incoherent traversals and loses where pops are frequent.
+        // The builder puts a child in the slot of the node corner it lies toward (bit a: high end of
+        // axis a), so a ray whose direction signs are r.neg meets them roughly in the order
+        // slot = i ^ r.neg, i = 0..7 (the ordering of compressed wide BVHs, Ylitie, Karras and
+        // Laine 2017); the hit mask is permuted into that order by three conditional bit-group
+        // swaps, and no distances are sorted.
+        const float tlim = __uint_as_float(uint32_t(min(r.klim, 0x7F800000))); // the limit as a distance
+        uint32_t hm = 0u; // bit c: slot c is hit
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint32_t sh = 8u * uint32_t(c & 3);
-        const float NX = __builtin_fmaf(float(((c < 4 ? nx0 : nx1) >> sh) & 0xFFu), ax, bx);
-        const float FX = __builtin_fmaf(float(((c < 4 ? fx0 : fx1) >> sh) & 0xFFu), ax, bx);
-        const float NY = __builtin_fmaf(float(((c < 4 ? ny0 : ny1) >> sh) & 0xFFu), ay, by);
-        const float FY = __builtin_fmaf(float(((c < 4 ? fy0 : fy1) >> sh) & 0xFFu), ay, by);
-        const float NZ = __builtin_fmaf(float(((c < 4 ? nz0 : nz1) >> sh) & 0xFFu), az, bz);
-        const float FZ = __builtin_fmaf(float(((c < 4 ? fz0 : fz1) >> sh) & 0xFFu), az, bz);
-        const float tn = fmaxf(fmaxf(NX, NY), fmaxf(NZ, r.t0));
-        const float tf = fminf(fminf(FX, FY), fminf(FZ, tlim));
-        const uint32_t code = ((c < 4 ? h1.z : h1.w) >> sh) & 0xFFu;
-        hm |= (tn <= tf && code != BVH8_EMPTY) ? (1u << c) : 0u;
+        for (int c = 0; c < 8; c++) hm |= tn[c] <= fminf(tf[c], tlim) ? (1u << c) : 0u;
+        // position i of the visiting order is slot i ^ neg: swap bit pairs, pairs of pairs, nibbles
+        uint32_t pm = hm;
+        if (r.neg & 1u) pm = ((pm & 0x55u) << 1) | ((pm >> 1) & 0x55u);
+        if (r.neg & 2u) pm = ((pm & 0x33u) << 2) | ((pm >> 2) & 0x33u);
+        if (r.neg & 4u) pm = ((pm & 0x0Fu) << 4) | (pm >> 4);
+        if (pm == 0u) {
+            r.cur = pop_next(bvh, r, stk);
+            return;
+        }
+        const uint32_t rest = pm & (pm - 1u);
+        if (rest != 0u) stack_push(stk, r.sp, r.cur | (rest << 24));
+        const uint32_t c = uint32_t(__builtin_ctz(pm)) ^ r.neg;
+        r.cur = code_entry(n.child_base, n.tri_base, __builtin_amdgcn_perm(n.code[1], n.code[0], c | 0x0C0C0C00u));
     }
-    // position i of the visiting order is slot i ^ neg: swap bit pairs, pairs of pairs, nibbles
-    uint32_t pm = hm;
-    if (r.neg & 1u) pm = ((pm & 0x55u) << 1) | ((pm >> 1) & 0x55u);
-    if (r.neg & 2u) pm = ((pm & 0x33u) << 2) | ((pm >> 2) & 0x33u);
-    if (r.neg & 4u) pm = ((pm & 0x0Fu) << 4) | (pm >> 4);
-    if (pm == 0u) {
-        r.cur = pop_next<SL>(bvh, r, stk);
-        return;
-    }
-    const uint32_t rest = pm & (pm - 1u);
-    if (rest != 0u) stack_push<SL>(stk, r.sp, r.cur | (rest << 24));
-    r.cur = bvh8_entry(h1, uint32_t(__builtin_ctz(pm)) ^ r.neg);
 }
 
 // Moves a leaf entry in `cur` into the (empty) postponed slot and takes the next entry, so the
 // lane can keep stepping through inner nodes while its leaf waits for the wave's next leaf
 // phase (speculative traversal, Aila & Laine 2009).
-template <int SL, class BVH>
+template <class BVH>
 __device__ __forceinline__ void postpone_leaf(const BVH& bvh, RayState& r, const LaneStack& stk) {
     if (r.leaf == TRAVERSAL_DONE && is_leaf(r.cur)) {
         r.leaf = r.cur;
-        r.cur = pop_next<SL>(bvh, r, stk);
+        r.cur = pop_next(bvh, r, stk);
     }
 }
 
@@ -438,10 +382,10 @@ __device__ __forceinline__ void postpone_leaf(const BVH& bvh, RayState& r, const
 // guided chunks of (unclaimed rays) / (2 * waves), 64..1024 rays, from `work`.
 // Refilled lanes issue their ray loads before the still-active lanes' traversal step, so both
 // wait on one memory round trip.
-template <int SL, bool COUNT, class Src, class Sink, bool ANY = false, class BVH = DeviceBVH>
+template <bool COUNT, bool ANY, class Src, class Sink, class BVH>
 __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, const Sink& sink, uint32_t n,
                                                  uint32_t* work, uint32_t ray_mask, const LaneStack& stk,
-                                                 TraversalCount& count, uint32_t refill, uint32_t leaf_lanes) {
+                                                 TraversalCount& count, uint32_t refill, uint32_t leaf_lanes, float dir_min) {
     const uint32_t lane = __lane_id();
     const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -507,19 +451,19 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
         if ((mi | ml) == 0 && __ballot(fresh) == 0) break;
         const bool leaf_phase = mi == 0 || uint32_t(__popcll(ml & ~mi)) >= leaf_lanes;
         if (leaf_phase) {
-            if (has_leaf) leaf_test<SL, COUNT, ANY>(bvh.tris, r, ray_mask, count);
+            if (has_leaf) leaf_test<COUNT, ANY>(bvh.tris, r, ray_mask, count);
         } else {
-            if (inner_ok) node_step<SL, COUNT>(bvh, r, stk, count);
+            if (inner_ok) node_step<COUNT>(bvh, r, stk, count);
         }
         if (active) {
-            postpone_leaf<SL>(bvh, r, stk);
+            postpone_leaf(bvh, r, stk);
             if (r.cur == TRAVERSAL_DONE && r.leaf == TRAVERSAL_DONE) {
                 sink.store(idx, r.best);
                 active = false;
             }
         }
         if (fresh) {
-            ray_begin(r, r.o, r.d, r.tmin, r.tmax);
+            ray_begin(r, r.o, r.d, r.tmin, r.tmax, dir_min);
             active = true;
         }
     }

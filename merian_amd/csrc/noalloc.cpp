@@ -69,8 +69,7 @@ MRT_API mrt_status mrt_trace_closest_noalloc_dev(mrt_ctx* c, mrt_scene* s, const
         if (c->device >= 0 && c->device < MAX_DEVICES) base = g_scratch_ptr[c->device];
     }
     if (!base) return fail(c, MRT_ERR_DEVICE, "mrt_trace_closest_noalloc_dev: scratch not set up on this device");
-    const uint32_t need = s->ds.stack_need;
-    const uint64_t entries = need > uint32_t(TRACE_LDS_STACK) ? need - TRACE_LDS_STACK : 1u;
+    const uint64_t entries = trace_ovf_entries(s->ds.stack_need);
     uint64_t threads = (SCRATCH_WORDS - CURSOR_WORDS) / entries / TRACE_BLOCK * TRACE_BLOCK;
     if (threads > trace_max_threads()) threads = trace_max_threads();
     if (threads < uint64_t(TRACE_BLOCK))

@@ -117,8 +117,7 @@ JobShape shape_of(const mrt_server* s, const mrt_job_desc& d) {
     sh.demod = d.params.demodulate_albedo != 0;
     sh.max_paths = sh.nee ? std::min<uint64_t>(s->cfg.max_paths_per_job, NEE_MAX_PATHS) : s->cfg.max_paths_per_job;
     sh.trace_threads = s->trace_threads;
-    const uint32_t need = d.scene->ds.stack_need;
-    sh.stack_entries = need > uint32_t(TRACE_LDS_STACK) ? need - TRACE_LDS_STACK : 1u;
+    sh.stack_entries = trace_ovf_entries(d.scene->ds.stack_need);
     return sh;
 }
 

@@ -29,10 +29,13 @@ mrt_status rebuild_bvh(mrt_ctx* c, mrt_scene* s, uint32_t width, uint32_t max_le
     const void* tri_src;
     size_t node_bytes, tri_bytes, n_nodes;
     uint32_t depth;
+    float dir_min;
     BVH4 b4;
     BVH8 b8;
     if (width == 8) {
         b8 = build_bvh8(v0, e1, e2, fl, n, 0, int(max_leaf), traversal_cost);
+        b8.tris.resize(b8.tris.size() + TRI_PADDING);
+        dir_min = bvh_dir_min(b8.max_exp);
         node_src = b8.nodes.data();
         node_bytes = b8.nodes.size() * sizeof(BVH8Node);
         n_nodes = b8.nodes.size();
@@ -41,6 +44,8 @@ mrt_status rebuild_bvh(mrt_ctx* c, mrt_scene* s, uint32_t width, uint32_t max_le
         depth = b8.depth;
     } else {
         b4 = build_bvh4(v0, e1, e2, fl, n, 0, int(max_leaf), traversal_cost);
+        b4.tris.resize(b4.tris.size() + TRI_PADDING);
+        dir_min = bvh_dir_min(b4.max_exp);
         node_src = b4.nodes.data();
         node_bytes = b4.nodes.size() * sizeof(BVH4Node);
         n_nodes = b4.nodes.size();
@@ -83,6 +88,7 @@ mrt_status rebuild_bvh(mrt_ctx* c, mrt_scene* s, uint32_t width, uint32_t max_le
     s->bytes += node_bytes + tri_bytes;
     // at most width - 1 entries per level (a grouped BVH8 traversal needs one)
     s->ds.stack_need = (width - 1u) * depth + 4u;
+    s->ds.dir_min = dir_min;
     s->n_nodes = n_nodes;
     s->depth = depth;
     s->tuning.bvh_width = width;

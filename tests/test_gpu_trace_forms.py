@@ -1,0 +1,86 @@
+"""Closest hits for the forms of rays and scenes at which the box tests' number formats could go
+wrong, bit-exact against the oracle's brute force on every tree: geometry far from the origin, tiny
+and huge, negative; rays along the axes and with zero components, directions of any length, intervals
+that start below zero, end at zero or are empty; odd ray counts from a single ray up; no triangles."""
+import numpy as np
+import pytest
+
+from merian_amd import abi, scenes
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TREES = [(4, 4, 0), (4, 1, 0), (8, 2, 0), (8, 2, 1)]
+
+
+def _scene(ctx, pos, idx, tree):
+    ds = ctx.triangles(pos, idx)
+    t = ds.tuning()
+    t.bvh_width, t.bvh_max_leaf, t.bvh8_order = tree
+    ds.set_tuning(t)
+    return ds
+
+
+def _same(a, b):
+    assert np.array_equal(a["triangle"], b["triangle"]), int((a["triangle"] != b["triangle"]).sum())
+    hit = b["triangle"] != 0xFFFFFFFF
+    for k in ("t", "u", "v"):
+        assert np.array_equal(a[k][hit].view(np.uint32), b[k][hit].view(np.uint32)), k
+    return hit
+
+
+def _rays(n, seed, scale, shift):
+    r = scenes.incoherent_rays(n, seed=seed)
+    r["origin"] = (r["origin"] * np.float32(scale) + np.float32(shift)).astype(np.float32)
+    d = r["direction"]
+    k = np.arange(n)
+    d[k % 7 == 0] = np.eye(3, dtype=np.float32)[k[k % 7 == 0] % 3] * np.where(k[k % 7 == 0] % 2, 1, -1)[:, None]
+    d[k % 7 == 1, 0] = 0.0
+    d[k % 7 == 2, 1] = -0.0
+    d[k % 7 == 3] *= np.float32(1e-4)
+    d[k % 7 == 4] *= np.float32(1e3)
+    r["tmax"][k % 11 == 0] = np.float32(0.3 * scale)
+    r["tmin"][k % 11 == 1] = np.float32(-0.5 * scale)
+    r["tmax"][k % 11 == 2] = -0.0
+    r["tmin"][k % 11 == 3], r["tmax"][k % 11 == 3] = np.float32(scale), np.float32(0.5 * scale)
+    r["tmin"][k % 11 == 4], r["tmax"][k % 11 == 4] = np.float32(-scale), np.float32(-0.01 * scale)
+    return r
+
+
+@pytest.mark.parametrize("tree", TREES)
+@pytest.mark.parametrize("scale,shift", [(1.0, 0.0), (1.0, -0.5), (1e-3, -0.25), (1e-2, 40.0), (1e5, -3e4), (1e8, 0.0)])
+def test_forms_vs_bruteforce(ctx, tree, scale, shift):
+    pos, idx = scenes.ray_query(seed=9, n_tri=1500)
+    pos = (pos * np.float32(scale) + np.float32(shift)).astype(np.float32)
+    rays = _rays(6001, 4, scale, shift)
+    ref = O.OracleScene(triangles=(pos, idx), use_bvh=False).trace(rays)
+    ds = _scene(ctx, pos, idx, tree)
+    got = ctx.trace(ds, rays)
+    ds.destroy()
+    assert _same(got, ref).mean() > 0.1
+
+
+@pytest.mark.parametrize("tree", TREES)
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1000, 16385, 400_003])
+def test_ray_counts(ctx, tree, n):
+    pos, idx = scenes.ray_query(seed=3, n_tri=3000)
+    rays = scenes.incoherent_rays(n, seed=5)
+    ref = O.OracleScene(triangles=(pos, idx), use_bvh=True).trace(rays)
+    ds = _scene(ctx, pos, idx, tree)
+    for _ in range(2):
+        _same(ctx.trace(ds, rays), ref)
+    ds.destroy()
+
+
+@pytest.mark.parametrize("tree", TREES)
+def test_no_triangles_and_one(ctx, tree):
+    rays = _rays(500, 1, 1.0, 0.0)
+    tri = np.array([[0.1, 0.1, 0.5], [0.9, 0.1, 0.5], [0.5, 0.9, 0.5]], np.float32)
+    for idx in (np.zeros(0, np.uint32), np.arange(3, dtype=np.uint32)):
+        ds = _scene(ctx, tri, idx, tree)
+        got = ctx.trace(ds, rays)
+        ds.destroy()
+        if len(idx):
+            _same(got, O.OracleScene(triangles=(tri, idx), use_bvh=False).trace(rays))
+        else:
+            assert (got["triangle"] == 0xFFFFFFFF).all()
