@@ -59,6 +59,10 @@ inline uint32_t trace_ovf_entries(uint32_t need) {
 }
 // Threads per block of the trace kernels (also the LDS stack's column stride).
 constexpr int TRACE_BLOCK = 128;
+// Lanes launched per ray while the grid is not full: a wave's rays are spread over its lanes
+// (mrt_trace.h), so a launch of few rays starts with 64 / TRACE_SPREAD rays per wave (4, 8 and 16
+// measured alike).
+constexpr uint32_t TRACE_SPREAD = 8;
 
 // Per-context scratch of the trace kernels: the global part of the traversal stacks (`entries`
 // per thread, `threads` columns) and a ray cursor for launches that do not bring their own.

@@ -372,40 +372,188 @@ __device__ __forceinline__ void postpone_leaf(const BVH& bvh, RayState& r, const
     }
 }
 
+// What the lanes of a wave keep in LDS beside their stacks. Slot k belongs to the ray that lane k
+// loaded last; it is used once lanes share rays (trace_persistent).
+struct WaveShared {
+    unsigned long long key[64]; // closest hit of the ray so far: ordered t, then id (hit_key)
+    float t[64], u[64], v[64];  // that hit
+    uint32_t workers[64];       // lanes working on the ray
+    uint32_t giver[64];         // k-th lane that gives a stack entry away
+};
+
+// Idle lanes of a wave without fresh rays before they take work from the others (4, 16 and 32 measured
+// within 1 % of each other).
+constexpr uint32_t SHARE_IDLE = 16;
+
+// (t, id) as one integer that orders hits as the traversal does: smaller t first (-0 is 0), ties to
+// the lower id; a miss (t = inf, id = ~0) last.
+__device__ __forceinline__ unsigned long long hit_key(const HitRec& h) {
+    const uint32_t b = __float_as_uint(h.t + 0.0f);
+    return (static_cast<unsigned long long>(b ^ ((b >> 31) ? 0xFFFFFFFFu : 0x80000000u)) << 32) | h.id;
+}
+
+// LDS traffic between the lanes of one wave: the hardware keeps it in order; this keeps the compiler
+// from moving accesses across.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Rank of a lane among the lanes of a set.
+__device__ __forceinline__ uint32_t lane_rank(uint64_t mask, uint32_t lane) {
+    return uint32_t(__popcll(mask & ((1ull << lane) - 1ull)));
+}
+
+// After a leaf test in a shared wave: the lane's hit goes to its ray's slot if it is the closest so
+// far, and the ray's closest hit comes back as the limit of the lane's further tests.
+// found: the test found the lane's hit (its u and v are then the lane's own).
+template <bool ANY>
+__device__ __forceinline__ void share_hit(WaveShared& ws, RayState& r, uint32_t slot, bool found) {
+    const unsigned long long key = hit_key(r.best);
+    if (found) atomicMin(&ws.key[slot], key);
+    wave_fence();
+    const unsigned long long now = ws.key[slot];
+    if (now == key) {
+        if (found) {
+            ws.t[slot] = r.best.t;
+            ws.u[slot] = r.best.u;
+            ws.v[slot] = r.best.v;
+        }
+    } else {
+        // another lane's hit is closer: its (t, id) bounds this lane's tests (u and v stay in the slot)
+        const uint32_t b = uint32_t(now >> 32);
+        r.best.t = __uint_as_float(b ^ ((b >> 31) ? 0x80000000u : 0xFFFFFFFFu));
+        r.best.id = uint32_t(now);
+        r.klim = key_limit(r.tmax, r.best.t);
+    }
+    if constexpr (ANY) {
+        if (r.best.id != TRAVERSAL_DONE) {
+            r.cur = TRAVERSAL_DONE;
+            r.sp = 0;
+        }
+    }
+}
+
 // Persistent closest-hit loop of one wave: every lane runs one traversal step per iteration and,
 // when its ray is done, hands the hit to `sink` and later takes a fresh ray from `src`, so lanes
 // with short rays do not idle while others finish long ones.
 //
 // Ray indices are handed out in wave-private chunks, so the single device-wide cursor `work`
-// (zero at launch) sees a few atomics per wave instead of one per refill: every wave first owns
-// a static chunk of n / (2 * waves) rays (rounded down to whole waves of 64), then claims
-// guided chunks of (unclaimed rays) / (2 * waves), 64..1024 rays, from `work`.
+// (zero at launch) sees a few atomics per wave instead of one per refill (it takes 117 M a second):
+// every wave first owns a static chunk of n / (2 * waves) rays (rounded down to whole waves of 64),
+// then claims guided chunks of (unclaimed rays) / (2 * waves), 64..1024 rays, from `work`. A SHARE
+// launch has so few rays per wave that the claims would be its longest part: seven eighths of its
+// rays are owned, in batches of 64 that go round the waves (neighbouring camera rays cost alike: a
+// contiguous range per wave makes the 1080p GBuffer pass 566 us instead of 440), and with at most
+// 64 rays per wave all are, evenly.
 // Refilled lanes issue their ray loads before the still-active lanes' traversal step, so both
 // wait on one memory round trip.
-template <bool COUNT, bool ANY, class Src, class Sink, class BVH>
+//
+// Sharing (SHARE): once a wave has no fresh rays left, idle lanes take stack entries from lanes that
+// still have some and work on those rays too, so the end of a launch, and all of a small one, is
+// as long as its longest ray's work spread over the wave and not as its longest ray. A lane's ray
+// is then named by a slot; leaf tests merge hits there (share_hit), and the last lane to finish work
+// on a ray stores its hit. The result is the same: the closest (t, id) over all leaves reached.
+// A wave whose refill threshold is 64 (it loads a batch when all its lanes are idle) shares every
+// batch (a 512x512 frame so tuned 796 -> 682 us).
+template <bool COUNT, bool ANY, bool SHARE, class Src, class Sink, class BVH>
 __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, const Sink& sink, uint32_t n,
-                                                 uint32_t* work, uint32_t ray_mask, const LaneStack& stk,
+                                                 uint32_t* work, uint32_t ray_mask, const LaneStack& stk, WaveShared& ws,
                                                  TraversalCount& count, uint32_t refill, uint32_t leaf_lanes, float dir_min) {
     const uint32_t lane = __lane_id();
     const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t c0 = (n / (2u * waves)) & ~63u;
-    const uint32_t dyn0 = c0 * waves; // <= n / 2: dynamic claims start here
-    uint32_t pool = wave * c0, pool_end = pool + c0;
+    uint32_t pool, pool_end, dyn0; // dynamic claims start at dyn0
+    uint32_t batches = 0, batch = 0; // SHARE: batches of 64 rays this wave owns, taken so far
+    if (SHARE && n <= 64u * uint64_t(waves)) {
+        const uint32_t each = (n + waves - 1u) / waves;
+        pool = uint32_t(min(uint64_t(wave) * each, uint64_t(n)));
+        pool_end = min(pool + each, n);
+        dyn0 = n;
+    } else if (SHARE) {
+        batches = uint32_t(uint64_t(n) * 7u / (uint64_t(waves) * (8u * 64u)));
+        dyn0 = batches * waves * 64u;
+        pool = pool_end = 0u;
+    } else {
+        const uint32_t c0 = (n / (2u * waves)) & ~63u;
+        dyn0 = c0 * waves; // <= n / 2
+        pool = wave * c0;
+        pool_end = pool + c0;
+    }
     uint32_t seen = dyn0;
     bool claims_done = dyn0 >= n;
     RayState r;
     r.cur = TRAVERSAL_DONE;
+    r.sp = 0;
     bool active = false;
+    bool sharing = false; // wave-uniform
+    uint32_t slot = lane;
     uint32_t idx = 0;
     while (true) {
         const uint64_t idle = __ballot(!active);
         const uint32_t nidle = uint32_t(__popcll(idle));
         bool fresh = false;
-        if (nidle >= refill && !(claims_done && pool == pool_end)) {
+        const bool more = !(claims_done && pool == pool_end) || (SHARE && batch < batches); // fresh rays for this wave
+        if (!(nidle >= refill && more)) {
+            // a wave that refills only when all its lanes are idle (refill 64) shares every batch
+            if (SHARE && (!more || refill >= 64u)) {
+                const bool can_give = active && r.sp > 0 && r.sp <= TRACE_LDS_STACK;
+                const uint64_t givers = __ballot(can_give);
+                if (nidle >= SHARE_IDLE && givers != 0) {
+                    if (!sharing) {
+                        sharing = true;
+                        if (active) {
+                            ws.key[lane] = hit_key(r.best);
+                            ws.t[lane] = r.best.t;
+                            ws.u[lane] = r.best.u;
+                            ws.v[lane] = r.best.v;
+                            ws.workers[lane] = 1u;
+                        }
+                    }
+                    const uint32_t pairs = min(nidle, uint32_t(__popcll(givers)));
+                    const uint32_t rank = lane_rank(can_give ? givers : idle, lane);
+                    const bool give = can_give && rank < pairs, take = !active && rank < pairs;
+                    if (give) ws.giver[rank] = lane;
+                    wave_fence();
+                    const uint32_t from = take ? ws.giver[rank] : lane;
+                    const f3 o{__shfl(r.o.x, int(from)), __shfl(r.o.y, int(from)), __shfl(r.o.z, int(from))};
+                    const f3 d{__shfl(r.d.x, int(from)), __shfl(r.d.y, int(from)), __shfl(r.d.z, int(from))};
+                    const float tmin = __shfl(r.tmin, int(from)), tmax = __shfl(r.tmax, int(from));
+                    const float bt = __shfl(r.best.t, int(from));
+                    const uint32_t bid = __shfl(r.best.id, int(from));
+                    const uint32_t gslot = __shfl(slot, int(from)), gidx = __shfl(idx, int(from));
+                    const int gsp = __shfl(r.sp, int(from));
+                    if (take) {
+                        // the giver's next entry, the nearest of its pending ones
+                        const uint32_t e = ((lds_u32)(stk.lds + (int(from) - int(lane))))[(gsp - 1) * TRACE_BLOCK];
+                        ray_begin(r, o, d, tmin, tmax, dir_min);
+                        r.best.t = bt;
+                        r.best.id = bid;
+                        r.klim = key_limit(tmax, bt);
+                        slot = gslot;
+                        idx = gidx;
+                        atomicAdd(&ws.workers[slot], 1u);
+                        active = true;
+                        if constexpr (BVH::SORTED) {
+                            r.cur = e;
+                        } else { // a group of children
+                            stack_push(stk, r.sp, e);
+                            r.cur = pop_next(bvh, r, stk);
+                        }
+                        postpone_leaf(bvh, r, stk);
+                    }
+                    if (give) r.sp--;
+                }
+            }
+        } else {
+            sharing = sharing && nidle < 64u; // all lanes idle: no slot is in use
             const uint32_t avail = pool_end - pool;
             uint32_t lo = 0, hi = 0;
-            if (avail < nidle && !claims_done) {
+            if (SHARE && avail < nidle && batch < batches) {
+                lo = (batch * waves + wave) * 64u;
+                hi = lo + 64u;
+                batch++;
+            } else if (avail < nidle && !claims_done) {
                 const uint32_t left = n - (seen < n ? seen : n);
                 const uint32_t chunk = min(max((left / (2u * waves)) & ~63u, 64u), 1024u);
                 const uint32_t leader = uint32_t(__ffsll((unsigned long long)idle) - 1);
@@ -420,7 +568,7 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
                 if (base + chunk >= n) claims_done = true;
             }
             if (!active) {
-                const uint32_t k = uint32_t(__popcll(idle & ((1ull << lane) - 1ull)));
+                const uint32_t k = lane_rank(idle, lane);
                 uint32_t my = TRAVERSAL_DONE;
                 if (k < avail) {
                     my = pool + k;
@@ -429,6 +577,7 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
                 }
                 if (my != TRAVERSAL_DONE) {
                     idx = my;
+                    slot = lane;
                     src.load(idx, r.o, r.d, r.tmin, r.tmax); // this lane's state is dead until ray_begin
                     fresh = true;
                 }
@@ -451,14 +600,26 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
         if ((mi | ml) == 0 && __ballot(fresh) == 0) break;
         const bool leaf_phase = mi == 0 || uint32_t(__popcll(ml & ~mi)) >= leaf_lanes;
         if (leaf_phase) {
-            if (has_leaf) leaf_test<COUNT, ANY>(bvh.tris, r, ray_mask, count);
+            if (has_leaf) {
+                const uint32_t before = r.best.id;
+                leaf_test<COUNT, ANY>(bvh.tris, r, ray_mask, count);
+                if (SHARE && sharing) share_hit<ANY>(ws, r, slot, r.best.id != before);
+            }
         } else {
             if (inner_ok) node_step<COUNT>(bvh, r, stk, count);
         }
         if (active) {
             postpone_leaf(bvh, r, stk);
             if (r.cur == TRAVERSAL_DONE && r.leaf == TRAVERSAL_DONE) {
-                sink.store(idx, r.best);
+                if (SHARE && sharing) {
+                    wave_fence();
+                    if (atomicSub(&ws.workers[slot], 1u) == 1u) {
+                        r.best = HitRec{uint32_t(ws.key[slot]), ws.t[slot], ws.u[slot], ws.v[slot]};
+                        sink.store(idx, r.best);
+                    }
+                } else {
+                    sink.store(idx, r.best);
+                }
                 active = false;
             }
         }
