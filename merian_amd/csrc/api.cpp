@@ -384,7 +384,12 @@ MRT_API mrt_status mrt_scene_create(mrt_ctx* c, const mrt_scene_desc* d, mrt_sce
                   : M.metalness >= 0.5f              ? SHADE_CLASS_METAL
                                                      : SHADE_CLASS_DIELECTRIC;
         }
-        const uint32_t geom_word = g | (uint32_t(cls) << TRI_SHADE_CLASS_SHIFT);
+        const uint32_t shade_word = uint32_t(G.material_id) | ((G.flags & MRT_GEOM_USE_ENV_MAP) ? TRI_SHADE_ENV : 0u) |
+                                    ((G.flags & MRT_GEOM_FLIP_FACING) ? TRI_SHADE_FLIP : 0u) |
+                                    ((G.flags & MRT_GEOM_FLAT_SHADING) ? TRI_SHADE_FLAT : 0u) |
+                                    ((G.flags & MRT_GEOM_HAS_TANGENTS) ? TRI_SHADE_TANGENTS : 0u) |
+                                    ((G.flags & MRT_GEOM_TWO_SIDED) ? TRI_SHADE_TWO_SIDED : 0u) |
+                                    (uint32_t(cls) << TRI_SHADE_CLASS_SHIFT);
         for (uint32_t p = 0; p < G.primitive_count; p++, gid++) {
             uint32_t vi[3];
             for (int k = 0; k < 3; k++) {
@@ -421,7 +426,7 @@ MRT_API mrt_status mrt_scene_create(mrt_ctx* c, const mrt_scene_desc* d, mrt_sce
                 const uint32_t uv = uint32_t(v.uv[0]) | (uint32_t(v.uv[1]) << 16);
                 std::memcpy(ts + 12 + k, &uv, 4);
             }
-            std::memcpy(ts + 15, &geom_word, 4);
+            std::memcpy(ts + 15, &shade_word, 4);
         }
     }
     const mrt_tuning defaults = mrt_scene{}.tuning;

@@ -19,8 +19,8 @@ struct DeviceScene {
     const float4* tris;          // TriRecord stream, leaf order
     const uint4* tri_verts;      // per global triangle id: 3 global vertex indices, geometry index
     const float4* tri_shade;     // per global triangle id, 64 B: (p0, n0), (p1, n1), (p2, n2),
-                                 // (uv0, uv1, uv2, geometry | shading class << 24); n = oct normal
-                                 // bits, uv = 2 x half bits
+                                 // (uv0, uv1, uv2, TRI_SHADE_* word); n = oct normal bits,
+                                 // uv = 2 x half bits
     const mrt_vertex* verts;     // PackedVertexData
     const mrt_geometry* geoms;   // GeometryData
     const uint32_t* geom_first;  // global id of each geometry's first triangle
@@ -48,7 +48,13 @@ enum : uint32_t {
     SHADE_CLASS_TRANSMISSIVE = 4, // OpenPBR with transmission
     SHADE_CLASSES = 5
 };
-constexpr uint32_t TRI_SHADE_GEOM_MASK = 0xFFFFFFu;
+// The record's last word: material entry, what shading needs of the geometry's flags, and the class,
+// so that a hit reaches its material without reading its geometry (one dependent gather less:
+// triangle record -> material; the 1920x1080 64-spp frame 168.4 -> 164.4 ms, a 957x541 16-spp NEE frame
+// 11.66 -> 11.52 ms).
+constexpr uint32_t TRI_SHADE_MATERIAL_MASK = 0xFFFFu;
+constexpr uint32_t TRI_SHADE_ENV = 1u << 16, TRI_SHADE_FLIP = 1u << 17, TRI_SHADE_FLAT = 1u << 18,
+                   TRI_SHADE_TANGENTS = 1u << 19, TRI_SHADE_TWO_SIDED = 1u << 20;
 constexpr uint32_t TRI_SHADE_CLASS_SHIFT = 24;
 
 // Entries of the per-lane traversal stack kept in LDS; deeper entries go to TraceScratch.ovf.
