@@ -37,14 +37,20 @@ mrt_status hip_fail(mrt_ctx* c, hipError_t e, const char* what) {
 
 void* dev_alloc(mrt_ctx* c, size_t bytes, mrt_status* st) {
     if (bytes == 0) bytes = 16;
+    if (c->in_use + bytes > c->budget) host_dev_release(c);
     if (c->in_use + bytes > c->budget) {
         *st = fail(c, MRT_ERR_BUDGET,
                    "HBM budget exceeded: " + std::to_string(c->in_use + bytes) + " > " + std::to_string(c->budget));
         return nullptr;
     }
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess && host_dev_release(c)) {
+        (void)hipGetLastError(); // (a launch would report it as its own)
+        e = hipMalloc(&p, bytes);
+    }
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         *st = fail(c, MRT_ERR_ALLOC, std::string("hipMalloc: ") + hipGetErrorString(e));
         return nullptr;
     }
@@ -63,6 +69,79 @@ void dev_free(mrt_ctx* c, void* p) {
     }
     const hipError_t e = hipFree(p);
     if (e != hipSuccess) c->err = std::string("hipFree: ") + hipGetErrorString(e);
+}
+
+bool host_dev_release(mrt_ctx* c) {
+    if (!c->host_dev || c->host_dev_busy) return false;
+    dev_free(c, c->host_dev);
+    c->host_dev = nullptr;
+    c->host_dev_bytes = 0;
+    return true;
+}
+
+HostCall::HostCall(mrt_ctx* c, size_t bytes, mrt_status* st) : c_(c) {
+    *st = MRT_OK;
+    if (bytes <= HOST_DEV_BYTES && !c->host_dev_busy) {
+        if (c->host_dev_bytes < bytes) {
+            host_dev_release(c);
+            c->host_dev = dev_alloc(c, bytes, st);
+            if (*st != MRT_OK) {
+                c->host_dev = nullptr;
+                return;
+            }
+            c->host_dev_bytes = bytes;
+        }
+        block_ = static_cast<char*>(c->host_dev);
+        kept_ = c->host_dev_busy = true;
+    } else {
+        block_ = static_cast<char*>(dev_alloc(c, bytes, st));
+    }
+    if (*st == MRT_OK && !c->host_pinned &&
+        hipHostMalloc(&c->host_pinned, HOST_PINNED_BYTES, hipHostMallocDefault) != hipSuccess) {
+        c->host_pinned = nullptr; // copies then go straight from the caller's pages
+        (void)hipGetLastError();
+    }
+}
+
+HostCall::~HostCall() {
+    if (kept_) {
+        c_->host_dev_busy = false;
+    } else {
+        dev_free(c_, block_);
+    }
+}
+
+void* HostCall::take(size_t bytes) {
+    void* p = block_ + used_;
+    used_ += round(bytes);
+    return p;
+}
+
+hipError_t HostCall::upload(void* d, const void* h, size_t bytes) {
+    if (c_->host_pinned && staged_ + bytes <= HOST_PINNED_BYTES) {
+        char* s = static_cast<char*>(c_->host_pinned) + staged_;
+        staged_ += round(bytes);
+        std::memcpy(s, h, bytes);
+        h = s;
+    }
+    return hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c_->stream);
+}
+
+hipError_t HostCall::download(void* h, const void* d, size_t bytes) {
+    if (c_->host_pinned && staged_ + bytes <= HOST_PINNED_BYTES && n_copies_ < 4) {
+        char* s = static_cast<char*>(c_->host_pinned) + staged_;
+        staged_ += round(bytes);
+        copies_[n_copies_++] = Copy{h, s, bytes};
+        h = s;
+    }
+    return hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, c_->stream);
+}
+
+hipError_t HostCall::finish() {
+    const hipError_t e = hipStreamSynchronize(c_->stream);
+    if (e == hipSuccess)
+        for (int k = 0; k < n_copies_; k++) std::memcpy(copies_[k].host, copies_[k].staged, copies_[k].bytes);
+    return e;
 }
 
 // NULL selects the context's own stream; hipStreamLegacy selects the HIP null stream (the
@@ -228,6 +307,8 @@ MRT_API mrt_status mrt_destroy(mrt_ctx* c) {
     for (auto& kv : c->sizes) (void)hipFree(kv.first);
     c->sizes.clear();
     if (c->scratch_event) (void)hipEventDestroy(c->scratch_event);
+    for (hipEvent_t e : c->events) (void)hipEventDestroy(e);
+    if (c->host_pinned) (void)hipHostFree(c->host_pinned);
     const bool destroyed = hipStreamDestroy(c->stream) == hipSuccess;
     delete c;
     return ok && destroyed ? MRT_OK : MRT_ERR_DEVICE;
@@ -635,23 +716,17 @@ MRT_API mrt_status mrt_trace_closest(mrt_ctx* c, mrt_scene* s, const mrt_ray* ra
     if (n == 0) return MRT_OK;
     mrt_status st = ensure_trace_scratch(c, s);
     if (st != MRT_OK) return st;
-    void* dr = dev_alloc(c, n * sizeof(mrt_ray), &st);
-    if (st != MRT_OK) return st;
-    void* dh = dev_alloc(c, n * sizeof(mrt_hit), &st);
-    if (st != MRT_OK) {
-        dev_free(c, dr);
-        return st;
-    }
+    HostCall call(c, HostCall::round(n * sizeof(mrt_ray)) + HostCall::round(n * sizeof(mrt_hit)), &st);
+    if (st != MRT_OK) return st; // (the traversal scratch is in place: nothing else is allocated below)
+    mrt_ray* dr = static_cast<mrt_ray*>(call.take(n * sizeof(mrt_ray)));
+    mrt_hit* dh = static_cast<mrt_hit*>(call.take(n * sizeof(mrt_hit)));
     hipError_t e = scratch_begin(c, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dr, rays, n * sizeof(mrt_ray), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess)
-        e = launch_trace_rays(s->ds, scene_scratch(c, s), static_cast<mrt_ray*>(dr), n, static_cast<mrt_hit*>(dh),
-                              c->stream);
+    if (e == hipSuccess) e = call.upload(dr, rays, n * sizeof(mrt_ray));
+    if (e == hipSuccess) e = launch_trace_rays(s->ds, scene_scratch(c, s), dr, n, dh, c->stream);
     if (e == hipSuccess) e = scratch_end(c, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(hits, dh, n * sizeof(mrt_hit), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    dev_free(c, dr);
-    dev_free(c, dh);
+    if (e == hipSuccess) e = call.download(hits, dh, n * sizeof(mrt_hit));
+    const hipError_t ef = call.finish(); // also drains what a failed call has enqueued
+    if (e == hipSuccess) e = ef;
     return e == hipSuccess ? MRT_OK : hip_fail(c, e, "mrt_trace_closest");
 }
 
@@ -755,6 +830,7 @@ mrt_status render_frame_dev(mrt_ctx* c, mrt_scene* s, const mrt_pt_params* prm, 
         a.guide_record_shift = shift;
     }
     FrameTiming t;
+    t.events = &c->events;
     uint64_t segs = 0;
     const hipStream_t strm = pick_stream(c, stream);
     unsigned long long* tc = nullptr;
@@ -811,50 +887,54 @@ MRT_API mrt_status mrt_pt_render_dev(mrt_ctx* c, mrt_scene* s, const mrt_pt_para
     return render_frame_dev(c, s, prm, cam, frame, w, h, gbuffer, irradiance, signature, stats, stream, nullptr);
 }
 
+static mrt_status render_frame_host(mrt_ctx* c, mrt_scene* s, const mrt_pt_params* prm, const mrt_camera* cam,
+                                    uint32_t frame, uint32_t w, uint32_t h, float* irradiance, uint32_t* signature,
+                                    mrt_packed_hit* gbuffer, mrt_pt_stats* stats) {
+    mrt_status st = MRT_OK;
+    const uint64_t npix = uint64_t(w) * h;
+    if (npix == 0) return MRT_OK;
+    HostCall call(c, 2 * HostCall::round(npix * 16) + HostCall::round(npix * 4), &st);
+    if (st != MRT_OK) return st;
+    mrt_packed_hit* dg = static_cast<mrt_packed_hit*>(call.take(npix * sizeof(mrt_packed_hit)));
+    float* dout = static_cast<float*>(call.take(npix * 16));
+    uint32_t* dsig = static_cast<uint32_t*>(call.take(npix * 4));
+    hipError_t e = hipSuccess;
+    if (stats) { // the pool's first two events: the gbuffer's start and end
+        while (c->events.size() < 2 && e == hipSuccess) {
+            hipEvent_t n = nullptr;
+            if ((e = hipEventCreate(&n)) == hipSuccess) c->events.push_back(n);
+        }
+        if (e == hipSuccess) e = hipEventRecord(c->events[0], c->stream);
+        if (e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame events");
+    }
+    if (st == MRT_OK) st = mrt_gbuffer_dev(c, s, cam, w, h, prm->instance_mask, dg, nullptr);
+    if (st == MRT_OK && stats && (e = hipEventRecord(c->events[1], c->stream)) != hipSuccess)
+        st = hip_fail(c, e, "mrt_render_frame events");
+    if (st == MRT_OK) st = mrt_pt_render_dev(c, s, prm, cam, frame, w, h, dg, dout, signature ? dsig : nullptr, stats, nullptr);
+    if (st == MRT_OK && stats) {
+        e = hipEventSynchronize(c->events[1]);
+        if (e == hipSuccess) e = hipEventElapsedTime(&stats->ms_gbuffer, c->events[0], c->events[1]);
+        if (e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame gbuffer time");
+    }
+    if (st == MRT_OK) e = call.download(irradiance, dout, npix * 16);
+    if (st == MRT_OK && e == hipSuccess && signature) e = call.download(signature, dsig, npix * 4);
+    if (st == MRT_OK && e == hipSuccess && gbuffer) e = call.download(gbuffer, dg, npix * sizeof(mrt_packed_hit));
+    const hipError_t ef = call.finish();
+    if (e == hipSuccess) e = ef;
+    if (st == MRT_OK && e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame copy");
+    return st;
+}
+
 MRT_API mrt_status mrt_render_frame(mrt_ctx* c, mrt_scene* s, const mrt_pt_params* prm, const mrt_camera* cam,
                                     uint32_t frame, uint32_t w, uint32_t h, float* irradiance, uint32_t* signature,
                                     mrt_packed_hit* gbuffer, mrt_pt_stats* stats) {
     if (!c || !s || !cam || !irradiance) return fail(c, MRT_ERR_INVALID, "mrt_render_frame: null argument");
     mrt_status st = check_params(c, prm);
     if (st != MRT_OK) return st;
-    const uint64_t npix = uint64_t(w) * h;
-    if (npix == 0) return MRT_OK;
-    void* dg = dev_alloc(c, npix * sizeof(mrt_packed_hit), &st);
-    if (st != MRT_OK) return st;
-    void* dout = dev_alloc(c, npix * 16, &st);
-    void* dsig = st == MRT_OK ? dev_alloc(c, npix * 4, &st) : nullptr;
-    if (st == MRT_OK) {
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        hipError_t e = hipEventCreate(&e0);
-        if (e == hipSuccess) e = hipEventCreate(&e1);
-        if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
-        if (e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame events");
-        if (st == MRT_OK)
-            st = mrt_gbuffer_dev(c, s, cam, w, h, prm->instance_mask, static_cast<mrt_packed_hit*>(dg), nullptr);
-        if (st == MRT_OK && (e = hipEventRecord(e1, c->stream)) != hipSuccess) st = hip_fail(c, e, "mrt_render_frame events");
-        if (st == MRT_OK)
-            st = mrt_pt_render_dev(c, s, prm, cam, frame, w, h, static_cast<mrt_packed_hit*>(dg),
-                                   static_cast<float*>(dout), signature ? static_cast<uint32_t*>(dsig) : nullptr, stats,
-                                   nullptr);
-        if (st == MRT_OK && stats) {
-            e = hipEventSynchronize(e1);
-            if (e == hipSuccess) e = hipEventElapsedTime(&stats->ms_gbuffer, e0, e1);
-            if (e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame gbuffer time");
-        }
-        if (e0) (void)hipEventDestroy(e0);
-        if (e1) (void)hipEventDestroy(e1);
-        e = hipSuccess;
-        if (st == MRT_OK) e = hipMemcpyAsync(irradiance, dout, npix * 16, hipMemcpyDeviceToHost, c->stream);
-        if (st == MRT_OK && e == hipSuccess && signature)
-            e = hipMemcpyAsync(signature, dsig, npix * 4, hipMemcpyDeviceToHost, c->stream);
-        if (st == MRT_OK && e == hipSuccess && gbuffer)
-            e = hipMemcpyAsync(gbuffer, dg, npix * sizeof(mrt_packed_hit), hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (st == MRT_OK && e != hipSuccess) st = hip_fail(c, e, "mrt_render_frame copy");
-    }
-    dev_free(c, dg);
-    dev_free(c, dout);
-    dev_free(c, dsig);
+    st = render_frame_host(c, s, prm, cam, frame, w, h, irradiance, signature, gbuffer, stats);
+    // a kept block larger than this call needs may be what the frame's own buffers had no room for
+    if ((st == MRT_ERR_BUDGET || st == MRT_ERR_ALLOC) && host_dev_release(c))
+        st = render_frame_host(c, s, prm, cam, frame, w, h, irradiance, signature, gbuffer, stats);
     return st;
 }
 

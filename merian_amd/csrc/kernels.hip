@@ -1368,16 +1368,19 @@ template <bool COUNT, class Src, class Sink, bool ANY, int W, bool SHARE> int tr
 constexpr uint32_t SHARE_MAX_RAYS = 1u << 21;
 
 // Launches the persistent trace kernel over at most n_max rays (the actual count is *count_ptr
-// when given). `work` must be zero on entry.
+// when given). `work` must be zero on entry, or is cleared here (clear_work).
 template <bool COUNT, class Src, class Sink, bool ANY, int W, bool SHARE>
 hipError_t launch_trace_variant(const DeviceScene& s, const TraceScratch& ts, const Src& src, const Sink& sink,
                                 const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
-                                unsigned long long* counters, hipStream_t st) {
+                                unsigned long long* counters, hipStream_t st, bool clear_work) {
     const int resident = trace_resident_blocks<COUNT, Src, Sink, ANY, W, SHARE>();
     const int cap = std::max(1, int(int64_t(resident) * int64_t(ts.grid_pct) / 100));
     int g = grid_for(uint64_t(n_max) * (SHARE ? TRACE_SPREAD : 1u), TRACE_BLOCK, cap);
     if (uint64_t(g) * TRACE_BLOCK > ts.threads) g = int(ts.threads / TRACE_BLOCK);
     if (g <= 0) return hipErrorInvalidValue;
+    // a launch that owns all its rays statically never reads the cursor
+    if (clear_work && !(SHARE && uint64_t(n_max) <= uint64_t(g) * TRACE_BLOCK))
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, work, 1u);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_trace<COUNT, Src, Sink, ANY, W, SHARE>), dim3(g), dim3(TRACE_BLOCK), 0, st, s, src,
                        sink, count_ptr, n_max, work, mask, ts, counters);
     return hipGetLastError();
@@ -1385,25 +1388,25 @@ hipError_t launch_trace_variant(const DeviceScene& s, const TraceScratch& ts, co
 template <bool COUNT, class Src, class Sink, bool ANY, int W>
 hipError_t launch_trace_width(const DeviceScene& s, const TraceScratch& ts, const Src& src, const Sink& sink,
                               const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
-                              unsigned long long* counters, hipStream_t st) {
+                              unsigned long long* counters, hipStream_t st, bool clear_work) {
     if constexpr (!COUNT) { // the counting kernels count each ray's own traversal
         if (n_max <= SHARE_MAX_RAYS)
             return launch_trace_variant<COUNT, Src, Sink, ANY, W, true>(s, ts, src, sink, count_ptr, n_max, work, mask,
-                                                                        counters, st);
+                                                                        counters, st, clear_work);
     }
     return launch_trace_variant<COUNT, Src, Sink, ANY, W, false>(s, ts, src, sink, count_ptr, n_max, work, mask, counters,
-                                                                 st);
+                                                                 st, clear_work);
 }
 template <bool COUNT, class Src, class Sink, bool ANY = false>
 hipError_t launch_trace(const DeviceScene& s, const TraceScratch& ts, const Src& src, const Sink& sink,
                         const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
-                        unsigned long long* counters, hipStream_t st) {
+                        unsigned long long* counters, hipStream_t st, bool clear_work = false) {
     if (n_max == 0) return hipSuccess;
     if (s.stack_need > TRACE_LDS_STACK + ts.entries) return hipErrorInvalidValue; // overflow area too small
     if (s.width == 8 ? !s.nodes8 : !s.nodes) return hipErrorInvalidValue;
-    if (s.width != 8) return launch_trace_width<COUNT, Src, Sink, ANY, 4>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st);
-    return s.bvh8_order ? launch_trace_width<COUNT, Src, Sink, ANY, 9>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st)
-                        : launch_trace_width<COUNT, Src, Sink, ANY, 8>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st);
+    if (s.width != 8) return launch_trace_width<COUNT, Src, Sink, ANY, 4>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st, clear_work);
+    return s.bvh8_order ? launch_trace_width<COUNT, Src, Sink, ANY, 9>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st, clear_work)
+                        : launch_trace_width<COUNT, Src, Sink, ANY, 8>(s, ts, src, sink, count_ptr, n_max, work, mask, counters, st, clear_work);
 }
 
 // Launches of the shading kernels, with the full material tree (LAYERED) only for a scene that
@@ -1497,11 +1500,11 @@ hipError_t launch_trace_rays(const DeviceScene& s, const TraceScratch& ts, const
                              mrt_hit* hits, hipStream_t st, unsigned long long* counters) {
     if (n == 0) return hipSuccess;
     if (n > 0xFFFFFFFFull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, ts.work, 1u);
     if (counters)
         return launch_trace<true>(s, ts, SrcRays{rays}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu, counters,
-                                  st);
-    return launch_trace<false>(s, ts, SrcRays{rays}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu, nullptr, st);
+                                  st, true);
+    return launch_trace<false>(s, ts, SrcRays{rays}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu, nullptr, st,
+                               true);
 }
 
 hipError_t launch_running_mean(float4* acc, const float4* src, uint32_t n, uint32_t count, hipStream_t st) {
@@ -1522,9 +1525,8 @@ hipError_t launch_gbuffer(const DeviceScene& s, const TraceScratch& ts, const mr
     const uint64_t n = uint64_t(w) * h;
     if (n == 0) return hipSuccess;
     if (n > 0xFFFFFFFFull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, ts.work, 1u);
     return launch_trace<false>(s, ts, SrcCamera{cam, w, h}, SinkGBuffer{s.tri_verts, s.geom_first, out}, nullptr,
-                               uint32_t(n), ts.work, mask, nullptr, st);
+                               uint32_t(n), ts.work, mask, nullptr, st, true);
 }
 
 hipError_t launch_gbuffer_albedo(const DeviceScene& s, const mrt_camera& cam, uint32_t w, uint32_t h,
@@ -1568,19 +1570,38 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
     if (a.mode == MRT_MODE_NEE && uint64_t(a.npix) * chunk > NEE_MAX_PATHS) return hipErrorInvalidValue;
     const uint32_t n_chunks = (spp + chunk - 1) / chunk;
     const uint32_t per_chunk = uint32_t(L + 1);
-    // timing: one event before and after every launch, read once the frame has completed
-    std::vector<hipEvent_t> ev;
-    std::vector<int> kind; // per event pair: 0 trace, 1 shade
+    // timing: events before and after every timed launch, read once the frame has completed. A launch
+    // that follows another timed one starts at that one's end: one event less in the stream.
+    struct Span {
+        size_t begin, end;
+        int kind; // 0 trace, 1 shade
+    };
+    std::vector<Span> spans;
+    size_t n_ev = 2;      // events in use (the caller owns the first two)
+    bool at_end = false;  // the last event is the end of the launch just enqueued
     hipError_t terr = hipSuccess; // first timing failure: timing stops, the frame still renders
+    auto record = [&] {
+        std::vector<hipEvent_t>& pool = *timing->events;
+        while (pool.size() <= n_ev && terr == hipSuccess) {
+            hipEvent_t e;
+            terr = hipEventCreate(&e);
+            if (terr == hipSuccess) pool.push_back(e);
+        }
+        if (terr == hipSuccess) terr = hipEventRecord(pool[n_ev++], st);
+    };
+    // k < 0: a timed launch (or the frame) starts here; k >= 0: the launch of that kind ends here
     auto mark = [&](int k) {
         if (!timing || terr != hipSuccess) return;
-        hipEvent_t e;
-        terr = hipEventCreate(&e);
-        if (terr != hipSuccess) return;
-        ev.push_back(e);
-        terr = hipEventRecord(e, st);
-        if (k >= 0) kind.push_back(k);
+        if (k < 0) {
+            if (!at_end) record();
+        } else {
+            record();
+            spans.push_back(Span{n_ev - 2, n_ev - 1, k});
+        }
+        at_end = k >= 0;
     };
+    // a launch that is not timed is enqueued: the last event is no longer where the stream is
+    auto untimed = [&] { at_end = false; };
     mark(-1);
     if (a.demodulate) {
         if (!pb.demod) return hipErrorInvalidValue;
@@ -1602,6 +1623,7 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
         // BSDF mode shades the primary vertices per pixel (k_shade_primary); the other modes
         // seed the path queue and shade bounce 0 like every other bounce
         const bool fused_primary = a.mode == MRT_MODE_BSDF;
+        if (!fused_primary) untimed();
         if (mc) {
             hipLaunchKernelGGL(k_mcpg_init, dim3(grid_for(a.npix, 256, MAX_BLOCKS)), dim3(256), 0, st, s, a, gbuffer, pb,
                                cnt);
@@ -1654,6 +1676,7 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
                 mark(0);
             }
         }
+        untimed();
         if (guided && c == 0)
             hipLaunchKernelGGL(k_guide_targets, dim3(grid_for(pb.grec_cap, 256, MAX_BLOCKS)), dim3(256), 0, st, pb);
         hipLaunchKernelGGL(k_accumulate, dim3(grid_for(a.npix, 256, MAX_BLOCKS)), dim3(256), 0, st, a, pb,
@@ -1662,19 +1685,18 @@ hipError_t launch_pt_frame(const DeviceScene& s, const TraceScratch& ts, PtArgs 
     mark(-1);
     if (timing) {
         float ms_trace = 0.f, ms_shade = 0.f;
-        if (terr == hipSuccess) terr = hipEventSynchronize(ev.back());
-        // events: [frame start] then per launch (start, end) pairs, then [frame end]
-        for (size_t k = 0; k < kind.size() && terr == hipSuccess; k++) {
+        const std::vector<hipEvent_t>& ev = *timing->events;
+        if (terr == hipSuccess) terr = hipEventSynchronize(ev[n_ev - 1]);
+        timing->trace_launches = 0;
+        for (const Span& sp : spans) {
             float ms = 0.f;
-            terr = hipEventElapsedTime(&ms, ev[1 + 2 * k], ev[2 + 2 * k]);
-            (kind[k] == 0 ? ms_trace : ms_shade) += ms;
+            if (terr == hipSuccess) terr = hipEventElapsedTime(&ms, ev[sp.begin], ev[sp.end]);
+            (sp.kind == 0 ? ms_trace : ms_shade) += ms;
+            timing->trace_launches += sp.kind == 0;
         }
-        if (terr == hipSuccess) terr = hipEventElapsedTime(&timing->ms_total, ev.front(), ev.back());
+        if (terr == hipSuccess) terr = hipEventElapsedTime(&timing->ms_total, ev[2], ev[n_ev - 1]);
         timing->ms_trace = ms_trace;
         timing->ms_shade = ms_shade;
-        timing->trace_launches = 0;
-        for (int k : kind) timing->trace_launches += (k == 0);
-        for (auto& e : ev) (void)hipEventDestroy(e); // release; nothing to recover on failure
     }
     if (err != hipSuccess) return err;
     if (terr != hipSuccess) return terr;

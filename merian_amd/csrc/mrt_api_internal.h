@@ -24,6 +24,12 @@ struct mrt_ctx {
     // last launch that used the context's shared scratch (trace stacks and cursor, path buffers)
     hipEvent_t scratch_event = nullptr;
     hipStream_t scratch_stream = nullptr;
+    // device and pinned memory of the host-buffer entry points, kept between calls (HostCall)
+    void* host_dev = nullptr;
+    size_t host_dev_bytes = 0;
+    bool host_dev_busy = false;
+    void* host_pinned = nullptr; // HOST_PINNED_BYTES
+    std::vector<hipEvent_t> events; // timing events of frames that report statistics
 };
 
 struct mrt_scene {
@@ -45,6 +51,42 @@ mrt_status hip_fail(mrt_ctx* c, hipError_t e, const char* what);
 void* dev_alloc(mrt_ctx* c, size_t bytes, mrt_status* st);
 void dev_free(mrt_ctx* c, void* p);
 hipStream_t pick_stream(mrt_ctx* c, void* stream);
+
+// Device and staging memory of one call of a host-buffer entry point (which ends with the stream
+// drained). Calls of up to HOST_DEV_BYTES use one device block that the context keeps, instead of a
+// hipMalloc and a hipFree (a device synchronisation) per buffer and call; it is given back when
+// another allocation of the context does not fit, and at mrt_destroy. Copies of up to
+// HOST_PINNED_BYTES in all go through pinned memory. With the pooled timing events, measured from the
+// host: a closest-hit call of 1,500 rays 62 -> 58 us, a 160x90 frame with its G-buffer, signature and
+// statistics 364 -> 322 us; above the block's size the allocations are small beside the copies.
+constexpr size_t HOST_DEV_BYTES = size_t(64) << 20, HOST_PINNED_BYTES = size_t(1) << 20;
+class HostCall {
+  public:
+    // bytes: the sum of the call's device buffers, each rounded up to 256
+    HostCall(mrt_ctx* c, size_t bytes, mrt_status* st);
+    ~HostCall();
+    HostCall(const HostCall&) = delete;
+    HostCall& operator=(const HostCall&) = delete;
+    static size_t round(size_t b) { return (b + 255) & ~size_t(255); }
+    void* take(size_t bytes); // the next part of the block
+    hipError_t upload(void* d, const void* h, size_t bytes);
+    hipError_t download(void* h, const void* d, size_t bytes);
+    hipError_t finish(); // drains the stream, then hands out what was downloaded
+  private:
+    struct Copy {
+        void* host;
+        const void* staged;
+        size_t bytes;
+    };
+    mrt_ctx* c_;
+    char* block_ = nullptr;
+    size_t used_ = 0, staged_ = 0;
+    bool kept_ = false;
+    Copy copies_[4];
+    int n_copies_ = 0;
+};
+// Gives back the kept device block unless a call is using it; whether there was one.
+bool host_dev_release(mrt_ctx* c);
 mrt_status ensure_path_buffers(mrt_ctx* c, uint64_t paths, uint64_t npix, uint64_t counters);
 mrt_status check_params(mrt_ctx* c, const mrt_pt_params* p);
 mrt_status ensure_trace_scratch(mrt_ctx* c, const mrt_scene* s);

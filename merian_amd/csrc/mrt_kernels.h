@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "bvh.h"
 #include "../../include/merian_amd.h"
 
@@ -198,6 +200,8 @@ struct FrameTiming {
     float ms_trace = 0.f, ms_shade = 0.f, ms_total = 0.f;
     uint32_t trace_launches = 0;
     uint64_t shadow_rays = 0;
+    // events to time with, kept by the caller and added to on demand (the first two are the caller's own)
+    std::vector<hipEvent_t>* events = nullptr;
 };
 // One frame of pt over `gbuffer`; out = float4 irradiance per pixel; sig_out optional.
 // counters_host (optional) receives every chunk's queue sizes after the frame completes.
