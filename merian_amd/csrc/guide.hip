@@ -11,14 +11,22 @@ namespace mrt {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+
+// LDS traffic between the lanes of one wave: the hardware keeps it in order; this keeps the compiler
+// from moving accesses across.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 constexpr int GB = 256;        // threads per block (4 waves)
 constexpr int NT = 2;          // 16-query tiles per wave iteration
 constexpr int WQ = 16 * NT;    // queries per wave iteration
 constexpr int BQ = 4 * WQ;     // queries per block iteration
-constexpr int INT_ = 1;        // inference: 16-query tiles per wave iteration
-constexpr int IWQ = 16 * INT_;
-constexpr int IBQ = 4 * IWQ;
+constexpr int IB = 512;        // threads per inference block (8 waves)
+constexpr int IW = IB / 64;
+constexpr int I_TILES = 4;     // inference: most 16-query tiles per wave iteration
 
 __device__ __forceinline__ floatx4 mfma(const half8_t a, const half8_t b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -46,37 +54,23 @@ __device__ __forceinline__ float sh_coef(int k, float x, float y, float z) {
     }
 }
 
-// Corners of grid level l around normalised position pn: table indices and trilinear weights
-// (corner bit 0 = x, 1 = y, 2 = z). Both layouts keep a grid row along x in consecutive
-// entries: dense levels are x-major, and a hashed level places row (y, z) at an offset in
-// [0, table - side] drawn from a hash of (y, z) (multiply-high range reduction), so
-// idx[2r + 1] == idx[2r] + 1 < table and one 8-byte load fetches each x-edge of the cell.
-__device__ __forceinline__ void grid_corners(const GuideNet& net, int l, const float pn[3], uint32_t idx[8], float w[8]) {
+// One grid level as the lanes that encode it hold it. Both layouts keep a grid row along x in
+// consecutive entries: dense levels are x-major, and a hashed level places row (y, z) at an offset
+// in [0, table - side] drawn from a hash of (y, z) (multiply-high range reduction), so one 16-byte
+// load fetches the two entries of an x-edge of a cell.
+struct GridLevel {
+    const uint2* table;
+    float res;
+    int last;             // the last cell along an axis
+    uint32_t side, span;  // entries along an axis; row offsets (side <= table is checked at create)
+    bool dense;
+};
+
+__device__ __forceinline__ GridLevel grid_level(const GuideNet& net, int l) {
     const uint32_t res = net.res[l];
-    int ci[3];
-    float fr[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const float x = pn[a] * float(res);
-        int c = int(floorf(x));
-        c = c >= int(res) ? int(res) - 1 : (c < 0 ? 0 : c);
-        ci[a] = c;
-        fr[a] = x - float(c);
-    }
     const uint64_t side = uint64_t(res) + 1;
-    const bool dense = side * side * side <= uint64_t(net.table);
-    const uint32_t span = net.table - uint32_t(side) + 1u; // row offsets; side <= table (checked at create)
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint32_t cx = uint32_t(ci[0] + (c & 1)), cy = uint32_t(ci[1] + ((c >> 1) & 1)),
-                       cz = uint32_t(ci[2] + ((c >> 2) & 1));
-        idx[c] = dense ? uint32_t(cx + side * (cy + side * cz))
-                       : uint32_t((uint64_t((cy * 2654435761u) ^ (cz * 805459861u)) * span) >> 32) + cx;
-        const float wx = (c & 1) ? fr[0] : 1.f - fr[0];
-        const float wy = (c & 2) ? fr[1] : 1.f - fr[1];
-        const float wz = (c & 4) ? fr[2] : 1.f - fr[2];
-        w[c] = (wx * wy) * wz;
-    }
+    return GridLevel{reinterpret_cast<const uint2*>(net.grid) + size_t(l) * net.table, float(res), int(res) - 1,
+                     uint32_t(side), net.table - uint32_t(side) + 1u, side * side * side <= uint64_t(net.table)};
 }
 
 // One of those corners: its table index and weight.
@@ -128,28 +122,47 @@ __device__ __forceinline__ void add_entry(float f[4], float w, uint32_t lo, uint
     f[3] += w * half_to_float(uint16_t(hi >> 16));
 }
 
+// The four features of one grid level at normalised position pn: trilinear over the cell's corners.
+// The rows of the four x-edges are computed once for both of their corners, in 32 bits (a dense
+// level's indices are below the table's size).
+__device__ __forceinline__ void encode_level(const GridLevel& L, const float pn[3], _Float16 out[G_FEATS]) {
+    uint32_t ci[3];
+    float fr[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float x = pn[a] * L.res;
+        const int c = min(max(int(floorf(x)), 0), L.last);
+        ci[a] = uint32_t(c);
+        fr[a] = x - float(c);
+    }
+    const uint32_t hy = ci[1] * 2654435761u, hz = ci[2] * 805459861u;
+    const uint32_t row = L.side * (ci[1] + L.side * ci[2]), up = L.side * L.side;
+    const float wx[2] = {1.f - fr[0], fr[0]}, wy[2] = {1.f - fr[1], fr[1]}, wz[2] = {1.f - fr[2], fr[2]};
+    float f[G_FEATS] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t y = e & 1, z = e >> 1;
+        const uint32_t hashed = __umulhi((hy + y * 2654435761u) ^ (hz + z * 805459861u), L.span);
+        const uint32_t dense = row + (y ? L.side : 0u) + (z ? up : 0u);
+        const EntryPair v = *reinterpret_cast<const EntryPair*>(L.table + ((L.dense ? dense : hashed) + ci[0]));
+        add_entry(f, (wx[0] * wy[y]) * wz[z], v.a0, v.a1);
+        add_entry(f, (wx[1] * wy[y]) * wz[z], v.b0, v.b1);
+    }
+#pragma unroll
+    for (int k = 0; k < G_FEATS; k++) out[k] = _Float16(f[k]);
+}
+
 // Encoding of one query by lane group g: chunk 0 = grid levels g and 4 + g (four features
 // each), chunk 1 = SH coefficients 4g..4g+3, then zeros.
 __device__ __forceinline__ void encode(const GuideNet& net, f3 p, f3 wo, int g, half8_t x[2]) {
     float pn[3];
     normalise(net, p, pn);
-    const uint32_t* tab = reinterpret_cast<const uint32_t*>(net.grid);
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const int l = slot_level(g, h);
-        uint32_t idx[8];
-        float w[8];
-        grid_corners(net, l, pn, idx, w);
-        const uint32_t* lt = tab + size_t(l) * net.table * 2;
-        float f[4] = {0.f, 0.f, 0.f, 0.f};
+        _Float16 f[G_FEATS];
+        encode_level(grid_level(net, slot_level(g, h)), pn, f);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const EntryPair v = *reinterpret_cast<const EntryPair*>(lt + 2 * size_t(idx[2 * e]));
-            add_entry(f, w[2 * e], v.a0, v.a1);
-            add_entry(f, w[2 * e + 1], v.b0, v.b1);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; k++) x[0][4 * h + k] = _Float16(f[k]);
+        for (int k = 0; k < G_FEATS; k++) x[0][4 * h + k] = f[k];
     }
 #pragma unroll
     for (int s = 0; s < 4; s++) x[1][s] = _Float16(sh_coef(4 * g + s, wo.x, wo.y, wo.z));
@@ -176,7 +189,8 @@ __device__ __forceinline__ void layer_mfma(const half8_t* frag, int layer, const
     }
 }
 
-// D layout -> B operand of the next layer (ReLU, fp16).
+// D layout -> B operand of the next layer (fp16, ReLU). The maximum is taken of the converted pairs:
+// the same values as before the conversion, in a quarter of the instructions.
 template <int T = NT>
 __device__ __forceinline__ void relu_to_operand(const floatx4 (&acc)[T][4], half8_t (&x)[T][2]) {
 #pragma unroll
@@ -184,7 +198,11 @@ __device__ __forceinline__ void relu_to_operand(const floatx4 (&acc)[T][4], half
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int s = 0; s < 8; s++) x[t][c][s] = _Float16(fmaxf(acc[t][2 * c + (s >> 2)][s & 3], 0.f));
+            for (int s = 0; s < 8; s++) x[t][c][s] = _Float16(acc[t][2 * c + (s >> 2)][s & 3]);
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) x[t][c] = __builtin_elementwise_max(x[t][c], half8_t{});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -274,16 +292,31 @@ struct LobeSink {
     }
 };
 
-// Inference: one 16-query tile per wave iteration, the forward weights in LDS (the last layer's
-// rows permuted, out_row_of), 4 waves per block. LDS holds nothing else (40 KB: four blocks per
-// CU), a query's outputs stay in the registers of the lanes that computed them, and one tile
-// keeps the kernel within 128 registers without spills: four waves per SIMD hide the latency of
-// the hash-grid gathers. The grid is capped at the resident blocks (1024), so the weights are
-// staged once per block.
+// What the four lane groups need of a query, written by the one lane that read it.
+struct __attribute__((aligned(16))) QueryRow {
+    float pn[3]; // normalised position
+    uint32_t valid;
+    half8_t sh[2]; // 16 SH coefficients of the direction
+};
+
+// Inference: the forward weights in LDS (the last layer's rows permuted, out_row_of), 8 waves per
+// block, one 16-query tile in registers at a time, and a query's outputs stay in the registers of the
+// lanes that computed them. The grid is capped at the resident blocks (two per CU: 64 KB of LDS each),
+// so the weights are staged once per block.
+//
+// Bound by the grid gathers' way through the L1 (the addresser is busy 4/5 of the time: eight 16-byte
+// accesses per lane and tile) and, next, by the instructions issued; the matrix cores idle. What does
+// not depend on the lane group is not repeated by it: a wave reads up to 64 queries at once, one per
+// lane (position from the hit, normalisation, SH coefficients), and hands them to its tiles through LDS;
+// the constants of a lane's two grid levels stay in registers. One bounce of a 960x540 16-spp frame
+// takes 465 us, 525 with every lane group reading its queries and evaluating its own coefficients in a
+// divergent switch. More waves per SIMD (five, six) and mixed-precision FMAs in place of the
+// conversions of the gathered halves change nothing.
 template <class Q, class Sink>
-__global__ __launch_bounds__(GB) __attribute__((amdgpu_waves_per_eu(4))) void k_guide_infer(GuideNet net, Q q, Sink sink) {
+__global__ __launch_bounds__(IB) __attribute__((amdgpu_waves_per_eu(4))) void k_guide_infer(GuideNet net, Q q, Sink sink) {
     __shared__ half8_t frag[G_FRAGS * 64]; // 40 KB: forward fragments of all layers
-    for (int k = threadIdx.x; k < G_FRAGS * 64; k += GB) {
+    __shared__ QueryRow queries[IW][16 * I_TILES];
+    for (int k = threadIdx.x; k < G_FRAGS * 64; k += IB) {
         const int layer = k / (8 * 64);
         if (layer < G_LAYERS - 1) {
             frag[k] = net.frag_fwd[k];
@@ -297,31 +330,56 @@ __global__ __launch_bounds__(GB) __attribute__((amdgpu_waves_per_eu(4))) void k_
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
     const uint32_t n = q.n();
-    const uint32_t stride = gridDim.x * IBQ;
-    for (uint32_t base = blockIdx.x * IBQ + wave * IWQ; base < n; base += stride) { // wave-uniform
-        half8_t x[INT_][2];
-        floatx4 acc[INT_][4];
-        bool valid[INT_];
-#pragma unroll
-        for (int t = 0; t < INT_; t++) {
-            const uint32_t i = base + t * 16 + (lane & 15);
+    // tiles per wave iteration: the fewest iterations of up to I_TILES, then spread evenly over them
+    const uint32_t waves = gridDim.x * IW;
+    const uint32_t rounds = (n / 16 + (n % 16 != 0) + waves - 1) / waves;
+    const uint32_t iterations = max((rounds + I_TILES - 1) / I_TILES, 1u);
+    const uint32_t tiles = max((rounds + iterations - 1) / iterations, 1u);
+    const GridLevel levels[2] = {grid_level(net, slot_level(g, 0)), grid_level(net, slot_level(g, 1))};
+    QueryRow* rows = queries[wave];
+    const uint32_t stride = waves * 16 * tiles;
+    for (uint32_t base = (blockIdx.x * IW + wave) * 16 * tiles; base < n; base += stride) { // wave-uniform
+        {
+            const uint32_t i = base + lane;
             f3 p{0.f, 0.f, 0.f}, wo{0.f, 0.f, 1.f};
-            valid[t] = i < n && q.load(i, p, wo);
-            encode(net, p, wo, g, x[t]);
-        }
+            QueryRow r;
+            r.valid = uint32_t(lane) < 16 * tiles && i < n && q.load(i, p, wo);
+            normalise(net, p, r.pn);
 #pragma unroll
-        for (int layer = 0; layer < 4; layer++) {
-            layer_mfma<4, INT_>(frag, layer, x, acc, lane);
-            relu_to_operand<INT_>(acc, x);
+            for (int k = 0; k < 16; k++) {
+                float c = sh_coef(k, wo.x, wo.y, wo.z);
+                asm("" : "+v"(c)); // rounded to 32 bits first, as everywhere: no fused product and conversion
+                r.sh[k >> 3][k & 7] = _Float16(c);
+            }
+            rows[lane] = r;
         }
-        layer_mfma<3, INT_>(frag, 4, x, acc, lane);
+        wave_lds_fence();
+#pragma unroll 1
+        for (uint32_t t = 0; t < tiles && base + 16 * t < n; t++) {
+            const QueryRow& r = rows[16 * t + (lane & 15)];
+            const float pn[3] = {r.pn[0], r.pn[1], r.pn[2]};
+            const bool valid = r.valid != 0;
+            half8_t x[1][2];
+            floatx4 acc[1][4];
+            _Float16 f[2][G_FEATS];
+            encode_level(levels[0], pn, f[0]);
+            encode_level(levels[1], pn, f[1]);
 #pragma unroll
-        for (int t = 0; t < INT_; t++) {
+            for (int k = 0; k < 8; k++) x[0][0][k] = f[k >> 2][k & 3];
+            const half4_t sh = reinterpret_cast<const half4_t*>(r.sh)[g];
+            x[0][1] = half8_t{sh[0], sh[1], sh[2], sh[3], 0, 0, 0, 0};
+#pragma unroll
+            for (int layer = 0; layer < 4; layer++) {
+                layer_mfma<4, 1>(frag, layer, x, acc, lane);
+                relu_to_operand<1>(acc, x);
+            }
+            layer_mfma<3, 1>(frag, 4, x, acc, lane);
             float o[10];
 #pragma unroll
-            for (int k = 0; k < 10; k++) o[k] = acc[t][k >> 2][k & 3];
-            sink.store(base + t * 16 + (lane & 15), valid[t], o, g);
+            for (int k = 0; k < 10; k++) o[k] = acc[0][k >> 2][k & 3];
+            sink.store(base + 16 * t + (lane & 15), valid, o, g);
         }
+        wave_lds_fence(); // the tiles have read their rows
     }
 }
 
@@ -731,8 +789,8 @@ hipError_t launch_guide_infer_queue(const GuideNet& net, const DeviceScene& s, c
                                     hipStream_t st) {
     if (n_max == 0) return hipSuccess;
     const QueueQueries q{s, qo, qd, hits, count, n_max};
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_guide_infer<QueueQueries, LobeSink>), dim3(blocks_for(n_max, IBQ, 1024)),
-                       dim3(GB), 0, st, net, q, LobeSink{lobes});
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_guide_infer<QueueQueries, LobeSink>), dim3(blocks_for(n_max, 16 * IW, 512)),
+                       dim3(IB), 0, st, net, q, LobeSink{lobes});
     return hipGetLastError();
 }
 
@@ -740,7 +798,7 @@ hipError_t launch_guide_forward(const GuideNet& net, const float4* pos, const fl
                                 hipStream_t st) {
     if (n == 0) return hipSuccess;
     const ArrayQueries q{pos, wo, n};
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_guide_infer<ArrayQueries, RawSink>), dim3(blocks_for(n, IBQ, 1024)), dim3(GB),
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_guide_infer<ArrayQueries, RawSink>), dim3(blocks_for(n, 16 * IW, 512)), dim3(IB),
                        0, st, net, q, RawSink{out});
     return hipGetLastError();
 }
