@@ -12,6 +12,7 @@
 #include "mrt_trace.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace mrt {
@@ -1361,11 +1362,17 @@ template <bool COUNT, class Src, class Sink, bool ANY, int W, bool SHARE> int tr
 }
 
 // Rays up to which a launch shares rays between lanes. Below it the end of the launch is a large part
-// of it: 1,500 rays 110 -> 61 us a call, 100,003 rays 157 -> 56 us, the 1080p GBuffer pass (2.07 M
-// rays) 501 -> 425 us, a 512x512 4-spp frame (up to 1 M rays a launch) 798 -> 631 us. Beyond it the
-// kernels without the sharing code hold one more wave per SIMD: with sharing a 957x541 16-spp NEE frame
-// (8.3 M paths) takes 11.93 ms instead of 11.65 and a batch of serving jobs 39.5 ms instead of 37.5.
-constexpr uint32_t SHARE_MAX_RAYS = 1u << 21;
+// of it, and so are the claims from the cursor, the last 1.8 M rays of a launch without sharing going 64
+// at a time: 1,500 rays 110 -> 61 us a call, 100,003 rays 157 -> 56 us, the 1080p GBuffer pass (2.07 M
+// rays) 501 -> 425 us, a 512x512 4-spp frame (up to 1 M rays a launch) 798 -> 631 us; with the limit at
+// 2^22 instead of 2^21, frames of 2.2 to 3.7 M paths 2.88 -> 2.02 ms, 5.84 -> 4.10 ms and 1.87 -> 1.11 ms.
+// Beyond it the kernels without the sharing code hold one more wave per SIMD: with sharing a 957x541
+// 16-spp NEE frame (8.3 M paths) takes 11.93 ms instead of 11.65 and a batch of serving jobs 39.5 ms
+// instead of 37.5. The caller's rays come all at once, where a frame's thin out bounce by bounce, and
+// soups of triangles load the claims less: sharing takes 2.9 M incoherent rays in meshes of 5 k to
+// 400 k triangles from 473 to 256 and from 618 to 407 us, but 4.1 M camera rays in a million triangles
+// from 3.16 to 3.87 ms and 3.5 M incoherent ones in 200 k from 2.05 to 2.32: those launches share less.
+constexpr uint32_t SHARE_MAX_RAYS = 1u << 22, SHARE_MAX_CALLER_RAYS = 3u << 20;
 
 // Launches the persistent trace kernel over at most n_max rays (the actual count is *count_ptr
 // when given). `work` must be zero on entry, or is cleared here (clear_work).
@@ -1390,7 +1397,7 @@ hipError_t launch_trace_width(const DeviceScene& s, const TraceScratch& ts, cons
                               const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
                               unsigned long long* counters, hipStream_t st, bool clear_work) {
     if constexpr (!COUNT) { // the counting kernels count each ray's own traversal
-        if (n_max <= SHARE_MAX_RAYS)
+        if (n_max <= (std::is_same<Src, SrcRays>::value ? SHARE_MAX_CALLER_RAYS : SHARE_MAX_RAYS))
             return launch_trace_variant<COUNT, Src, Sink, ANY, W, true>(s, ts, src, sink, count_ptr, n_max, work, mask,
                                                                         counters, st, clear_work);
     }

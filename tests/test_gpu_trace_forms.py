@@ -89,20 +89,20 @@ def test_no_triangles_and_one(ctx, tree):
 @pytest.fixture(scope="module")
 def soup():
     pos, idx = scenes.ray_query(seed=21, n_tri=20_000)
-    rays = scenes.incoherent_rays((1 << 21) + 65, seed=22)
+    rays = scenes.incoherent_rays((3 << 20) + 65, seed=22)
     return pos, idx, rays, O.OracleScene(triangles=(pos, idx), use_bvh=True).trace(rays)
 
 
 @pytest.mark.parametrize("tree", [(4, 2, 0), (8, 2, 0), (8, 4, 1)])
 @pytest.mark.parametrize("refill,grid", [(1, 100), (16, 3), (64, 100), (64, 1), (63, 1)])
 def test_shared_rays_and_refill(ctx, soup, tree, refill, grid):
-    """Launches whose lanes share rays (up to 2^21 of them), with every kind of refill and few or many
+    """Launches whose lanes share rays (up to 3 << 20 of them), with every kind of refill and few or many
     rays per wave, and one just above that limit."""
     pos, idx, rays, ref = soup
     ds = _scene(ctx, pos, idx, tree)
     t = ds.tuning()
     t.refill_lanes, t.grid_percent, t.leaf_lanes = refill, grid, 64 if refill == 63 else 8
     ds.set_tuning(t)
-    for n in (17, 4097, 130_001, *([1 << 21, len(rays)] if grid == 100 else [])):
+    for n in (17, 4097, 130_001, *([3 << 20, len(rays)] if grid == 100 else [])):
         _same(ctx.trace(ds, rays[:n]), ref[:n])
     ds.destroy()
