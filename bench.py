@@ -211,7 +211,7 @@ def small_leg(ctx, frames: int = 64, retune: bool = False) -> dict:
     bytes_per_seg = (st_c.node_visits * node_bytes + st_c.triangle_tests * TRI_BYTES) / cont + RAY_IO_BYTES
     cont_timed = segs - frames * W * H
     avg_ms = ms_trace / max(1, launches)
-    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(tuning)}>", avg_ms, launches,
+    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(tuning)}, true>", avg_ms, launches,
                     bytes_per_seg * cont_timed / max(1, launches), SMALL_TRAFFIC,
                     match={"tuning": tuning, "workload": SMALL_WORKLOAD},
                     extra={"bytes_per_segment": round(bytes_per_seg, 1)})
@@ -544,7 +544,7 @@ def ray_query_leg(ctx, reps: int = 3, retune: bool = False) -> dict:
         nodes, tris = ctx.trace_count_dev(ds, d_r.data_ptr(), n, d_hits.data_ptr())
         ms = _time_rays(ctx, ds, d_r, n, d_hits, stream, reps)
         bytes_per_ray = (nodes * NODE_BYTES[settings["bvh_width"]] + tris * TRI_BYTES) / n + RAY_IO_BYTES
-        roof = roofline(f"k_trace<false, SrcRays, SinkHits, false, {trace_variant(settings)}>", ms, reps,
+        roof = roofline(f"k_trace<false, SrcRays, SinkHits, false, {trace_variant(settings)}, false>", ms, reps,
                         bytes_per_ray * n, os.path.join(ROOT, "profiles", f"k_trace_rays_{name}.traffic.json"),
                         match={"tuning": settings, "workload": f"ray_query {name}"})
         res[name] = {"mrays_per_s": round(n / ms / 1e3, 1), "ms_per_launch": round(ms, 3),
@@ -716,7 +716,7 @@ def main():
     cont_timed = segs - args.steps * W * H
     bytes_per_launch = bytes_per_seg * cont_timed / max(1, launches)
     avg_ms = ms_trace / max(1, launches)
-    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(ds.tuning().as_dict())}>", avg_ms, launches,
+    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(ds.tuning().as_dict())}, false>", avg_ms, launches,
                     bytes_per_launch, TRAFFIC_FILE,
                     match={"tuning": tuning, "workload": TRAFFIC_WORKLOAD},
                     extra={"bytes_per_segment": round(bytes_per_seg, 1), "node_bytes": node_bytes,
