@@ -85,7 +85,7 @@ struct RayState {
     f3 o, d;
     float ix, iy, iz, ox, oy, oz;
     float t0, tmin, tmax;
-    int klim;     // far limit of the box tests as a sort key (key_limit)
+    int klim;     // far limit of the box tests (far_limit)
     uint32_t neg; // bit k: direction component k is negative
     uint32_t psel[3]; // v_perm selector per axis: the near planes of children 0 and 1 (lo for a
                       // positive direction, hi for a negative one) as two zero-extended bytes;
@@ -99,17 +99,21 @@ struct RayState {
 __device__ __forceinline__ bool is_inner(uint32_t e) { return !(e & LEAF_FLAG); }
 __device__ __forceinline__ bool is_leaf(uint32_t e) { return e != TRAVERSAL_DONE && (e & LEAF_FLAG); }
 
-// Far limit of the box tests, min(tmax, best.t) widened by 2 ulp, as a sort key: a child is
-// visited while its key is at most this. Keys compare as signed integers, so non-negative
-// distances compare as they should and a negative one (a box around the origin of a ray with a
-// negative tmin) is below every limit; a negative limit (nothing can be hit) admits everything
-// and leaves the rejection to the triangle test.
-__device__ __forceinline__ int key_limit(float tmax, float t) {
-    const float lim = fminf(tmax, t) * 1.00000024f;
+// Far limit of the box tests: min(tmax, best.t) widened by 2 ulp. Octant order compares distances
+// and takes the limit's bits as they are (upwards also from a negative one: an interval of one
+// negative point keeps its boxes). Sorted order takes it as a sort key: a child is visited while its
+// key is at most this. Keys compare as signed integers, so non-negative distances compare as they
+// should and a negative one (a box around the origin of a ray with a negative tmin) is below every
+// limit; a negative limit admits everything and leaves the rejection to the triangle test.
+template <bool SORTED> __device__ __forceinline__ int far_limit(float tmax, float t) {
+    const float m = fminf(tmax, t);
+    if constexpr (!SORTED) return int(__float_as_uint(m + fabsf(m) * 2.4e-7f));
+    const float lim = m * 1.00000024f;
     return lim >= 0.f ? int(__float_as_uint(fabsf(lim)) | 0xFFu) : KEY_MISS - 1; // fabsf: -0 is 0
 }
 
 // dir_min: smallest magnitude of a direction component in the box tests (DeviceScene.dir_min).
+template <bool SORTED>
 __device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, float tmax, float dir_min) {
     r.o = o;
     r.d = d;
@@ -130,7 +134,7 @@ __device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, f
     r.tmax = tmax;
     r.t0 = tmin - fabsf(tmin) * 2.4e-7f;
     r.best = HitRec{TRAVERSAL_DONE, __builtin_inff(), 0.f, 0.f};
-    r.klim = key_limit(tmax, r.best.t);
+    r.klim = far_limit<SORTED>(tmax, r.best.t);
     r.psel[0] = (r.neg & 1u) ? 0x0C050C04u : 0x0C010C00u;
     r.psel[1] = (r.neg & 2u) ? 0x0C050C04u : 0x0C010C00u;
     r.psel[2] = (r.neg & 4u) ? 0x0C050C04u : 0x0C010C00u;
@@ -140,7 +144,7 @@ __device__ __forceinline__ void ray_begin(RayState& r, f3 o, f3 d, float tmin, f
 }
 
 // Tests the triangles of the postponed leaf (ANY: the first hit ends the traversal).
-template <bool COUNT, bool ANY>
+template <bool COUNT, bool ANY, bool SORTED>
 __device__ __forceinline__ void leaf_test(const float4* __restrict__ tris, RayState& r, uint32_t ray_mask,
                                           TraversalCount& count) {
     const uint32_t first = (r.leaf & 0x7FFFFFFFu) >> 3;
@@ -155,7 +159,7 @@ __device__ __forceinline__ void leaf_test(const float4* __restrict__ tris, RaySt
     }
     if constexpr (COUNT) count.tris += cnt;
     r.leaf = TRAVERSAL_DONE;
-    r.klim = key_limit(r.tmax, r.best.t);
+    r.klim = far_limit<SORTED>(r.tmax, r.best.t);
     if constexpr (ANY) {
         if (r.best.id != TRAVERSAL_DONE) {
             r.cur = TRAVERSAL_DONE;
@@ -341,7 +345,7 @@ __device__ __forceinline__ void node_step(const BVH bvh, RayState& r, const Lane
         // slot = i ^ r.neg, i = 0..7 (the ordering of compressed wide BVHs, Ylitie, Karras and
         // Laine 2017); the hit mask is permuted into that order by three conditional bit-group
         // swaps, and no distances are sorted.
-        const float tlim = __uint_as_float(uint32_t(min(r.klim, 0x7F800000))); // the limit as a distance
+        const float tlim = __uint_as_float(uint32_t(r.klim));
         uint32_t hm = 0u; // bit c: slot c is hit
 #pragma unroll
         for (int c = 0; c < 8; c++) hm |= tn[c] <= fminf(tf[c], tlim) ? (1u << c) : 0u;
@@ -407,7 +411,7 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask, uint32_t lane) {
 // After a leaf test in a shared wave: the lane's hit goes to its ray's slot if it is the closest so
 // far, and the ray's closest hit comes back as the limit of the lane's further tests.
 // found: the test found the lane's hit (its u and v are then the lane's own).
-template <bool ANY>
+template <bool ANY, bool SORTED>
 __device__ __forceinline__ void share_hit(WaveShared& ws, RayState& r, uint32_t slot, bool found) {
     const unsigned long long key = hit_key(r.best);
     if (found) atomicMin(&ws.key[slot], key);
@@ -424,7 +428,7 @@ __device__ __forceinline__ void share_hit(WaveShared& ws, RayState& r, uint32_t 
         const uint32_t b = uint32_t(now >> 32);
         r.best.t = __uint_as_float(b ^ ((b >> 31) ? 0x80000000u : 0xFFFFFFFFu));
         r.best.id = uint32_t(now);
-        r.klim = key_limit(r.tmax, r.best.t);
+        r.klim = far_limit<SORTED>(r.tmax, r.best.t);
     }
     if constexpr (ANY) {
         if (r.best.id != TRAVERSAL_DONE) {
@@ -526,10 +530,10 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
                     if (take) {
                         // the giver's next entry, the nearest of its pending ones
                         const uint32_t e = ((lds_u32)(stk.lds + (int(from) - int(lane))))[(gsp - 1) * TRACE_BLOCK];
-                        ray_begin(r, o, d, tmin, tmax, dir_min);
+                        ray_begin<BVH::SORTED>(r, o, d, tmin, tmax, dir_min);
                         r.best.t = bt;
                         r.best.id = bid;
-                        r.klim = key_limit(tmax, bt);
+                        r.klim = far_limit<BVH::SORTED>(tmax, bt);
                         slot = gslot;
                         idx = gidx;
                         atomicAdd(&ws.workers[slot], 1u);
@@ -602,8 +606,8 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
         if (leaf_phase) {
             if (has_leaf) {
                 const uint32_t before = r.best.id;
-                leaf_test<COUNT, ANY>(bvh.tris, r, ray_mask, count);
-                if (SHARE && sharing) share_hit<ANY>(ws, r, slot, r.best.id != before);
+                leaf_test<COUNT, ANY, BVH::SORTED>(bvh.tris, r, ray_mask, count);
+                if (SHARE && sharing) share_hit<ANY, BVH::SORTED>(ws, r, slot, r.best.id != before);
             }
         } else {
             if (inner_ok) node_step<COUNT>(bvh, r, stk, count);
@@ -624,7 +628,7 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
             }
         }
         if (fresh) {
-            ray_begin(r, r.o, r.d, r.tmin, r.tmax, dir_min);
+            ray_begin<BVH::SORTED>(r, r.o, r.d, r.tmin, r.tmax, dir_min);
             active = true;
         }
     }

@@ -61,6 +61,28 @@ def test_forms_vs_bruteforce(ctx, tree, scale, shift):
 
 
 @pytest.mark.parametrize("tree", TREES)
+@pytest.mark.parametrize("ahead", [True, False])
+def test_interval_of_one_point(ctx, tree, ahead):
+    """tmin = tmax = the hit's own distance, ahead of the origin and behind it: the limits of the box
+    tests are rounded outward on both sides, so the hit stays."""
+    pos, idx = scenes.ray_query(seed=11, n_tri=4000)
+    rays = scenes.incoherent_rays(20_001, seed=6)
+    osc = O.OracleScene(triangles=(pos, idx), use_bvh=False)
+    if not ahead:
+        rays["direction"] *= -1
+        rays["tmin"], rays["tmax"] = -np.inf, 0.0
+    first = osc.trace(rays)
+    t = np.where(first["triangle"] != 0xFFFFFFFF, first["t"], np.float32(-1.0 if not ahead else 1.0))
+    rays["tmin"] = rays["tmax"] = t
+    ref = osc.trace(rays)
+    ds = _scene(ctx, pos, idx, tree)
+    got = ctx.trace(ds, rays)
+    ds.destroy()
+    hit = _same(got, ref)
+    assert hit.mean() > 0.3 and (got["t"][hit] == t[hit]).all()  # 39.6 % of these rays hit (brute force)
+
+
+@pytest.mark.parametrize("tree", TREES)
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1000, 16385, 400_003])
 def test_ray_counts(ctx, tree, n):
     pos, idx = scenes.ray_query(seed=3, n_tri=3000)
