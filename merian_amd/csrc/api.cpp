@@ -215,7 +215,7 @@ mrt_status ensure_trace_scratch(mrt_ctx* c, const mrt_scene* s) {
     mrt_status st = MRT_OK;
     t.ovf = static_cast<uint32_t*>(dev_alloc(c, size_t(threads) * need * 4, &st));
     if (st != MRT_OK) return st;
-    t.work = static_cast<uint32_t*>(dev_alloc(c, 64, &st));
+    t.work = static_cast<uint32_t*>(dev_alloc(c, CURSOR_WORDS * 4, &st));
     if (st != MRT_OK) {
         dev_free(c, t.ovf);
         t = TraceScratch{};

@@ -74,6 +74,7 @@ __device__ __forceinline__ RayF camera_ray(const mrt_camera& c, uint32_t px, uin
 
 // Ray sources and hit sinks of the persistent traversal loop.
 struct SrcRays { // mrt_ray array: (origin, tmin), (direction, tmax)
+    static constexpr bool CURSORS = false;
     const mrt_ray* rays;
     __device__ __forceinline__ void load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax) const {
         const float4* rp = reinterpret_cast<const float4*>(rays + i);
@@ -84,7 +85,11 @@ struct SrcRays { // mrt_ray array: (origin, tmin), (direction, tmax)
         tmax = b.w;
     }
 };
+struct SrcSomeRays : SrcRays { // an array of CURSORS_MIN_RAYS to CURSORS_MAX_RAYS
+    static constexpr bool CURSORS = true;
+};
 struct SrcQueue { // path queue: (origin, path id), (direction, -); continuation rays [0, 1e7]
+    static constexpr bool CURSORS = false;
     const float4* qo;
     const float4* qd;
     __device__ __forceinline__ void load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax) const {
@@ -96,6 +101,7 @@ struct SrcQueue { // path queue: (origin, path id), (direction, -); continuation
     }
 };
 struct SrcCamera { // primary rays of a w x h image
+    static constexpr bool CURSORS = false;
     mrt_camera cam;
     uint32_t w, h;
     __device__ __forceinline__ void load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax) const {
@@ -140,6 +146,7 @@ struct SinkGBuffer { // PackedHitInfo (gbuffer.slang:175-196); one pretransforme
 };
 
 struct SrcShadow { // NEE shadow queue: (origin, radiance target), (direction, -); [0, 1e7] like a continuation ray
+    static constexpr bool CURSORS = false;
     const float4* so;
     const float4* sd;
     __device__ __forceinline__ void load(uint32_t i, f3& o, f3& d, float& tmin, float& tmax) const {
@@ -205,6 +212,7 @@ template <> constexpr int TRACE_WAVES<SrcQueue, 8> = 6;
 template <> constexpr int TRACE_WAVES<SrcShadow, 8> = 6;
 template <> constexpr int TRACE_WAVES<SrcRays, 8> = 5;
 template <> constexpr int TRACE_WAVES<SrcRays, 4> = 7;
+template <int W> constexpr int TRACE_WAVES<SrcSomeRays, W> = TRACE_WAVES<SrcRays, W>;
 // SHARE: idle lanes take work from others at the end (small launches, SHARE_MAX_RAYS).
 template <bool COUNT, class Src, class Sink, bool ANY = false, int W = 4, bool SHARE = false>
 __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHARE ? 1 : TRACE_WAVES<Src, W>))) void k_trace(DeviceScene S, Src src, Sink sink,
@@ -1364,18 +1372,30 @@ template <bool COUNT, class Src, class Sink, bool ANY, int W, bool SHARE> int tr
 // Rays up to which a launch shares rays between lanes. Below it the end of the launch is a large part
 // of it, and so are the claims from the cursor, the last 1.8 M rays of a launch without sharing going 64
 // at a time: 1,500 rays 110 -> 61 us a call, 100,003 rays 157 -> 56 us, the 1080p GBuffer pass (2.07 M
-// rays) 501 -> 425 us, a 512x512 4-spp frame (up to 1 M rays a launch) 798 -> 631 us; with the limit at
-// 2^22 instead of 2^21, frames of 2.2 to 3.7 M paths 2.88 -> 2.02 ms, 5.84 -> 4.10 ms and 1.87 -> 1.11 ms.
+// rays) 501 -> 404 us and one of 4.10 M pixels 905 -> 720, a 512x512 4-spp frame (up to 1 M rays a
+// launch) 798 -> 631 us; with the limit at 2^22 instead of 2^21, frames of 2.2 to 3.7 M paths
+// 2.88 -> 2.02 ms, 5.84 -> 4.10 ms and 1.87 -> 1.11 ms.
 // Beyond it the kernels without the sharing code hold one more wave per SIMD: with sharing a 957x541
 // 16-spp NEE frame (8.3 M paths) takes 11.93 ms instead of 11.65 and a batch of serving jobs 39.5 ms
-// instead of 37.5. The caller's rays come all at once, where a frame's thin out bounce by bounce, and
-// soups of triangles load the claims less: sharing takes 2.9 M incoherent rays in meshes of 5 k to
-// 400 k triangles from 473 to 256 and from 618 to 407 us, but 4.1 M camera rays in a million triangles
-// from 3.16 to 3.87 ms and 3.5 M incoherent ones in 200 k from 2.05 to 2.32: those launches share less.
+// instead of 37.5. A caller's rays have several cursors on both sides, so that the waves decide alone,
+// and earlier: at 3.3 M rays sharing takes 210 us instead of 247 in a mesh of 46 k
+// triangles, 1.83 ms instead of 2.22 for incoherent rays in 200 k triangles, and the same for camera
+// rays in a million (2.89, 2.88); at 6.0 M those take 4.97 ms instead of 4.31.
 constexpr uint32_t SHARE_MAX_RAYS = 1u << 22, SHARE_MAX_CALLER_RAYS = 3u << 20;
 
+// Sizes between which a caller's array is divided among several cursors. With batches and one cursor
+// such a launch waited for its claims or, in deep trees, lost more to the scattered rays of a wave than
+// the balance gained: 3.0 M camera rays in a million triangles 2.99 -> 2.75 ms (2.86 before lanes
+// shared rays), 2.2 M 2.31 -> 2.01 (2.22), 2.2 M in 200,000 triangles 1.02 -> 0.93 (0.96), 3.3 M
+// incoherent rays in a mesh of 46 k triangles 478 -> 248 us (450), 6.0 M 575 -> 383 (561). Below, the
+// batches are as good (1.0 M camera rays 1.04 ms, 1.08 halved). Above, the claims are a small part
+// (9.5 M rays in the mesh: 689 us, 747 before) and rays that stay together count more: 16.8 M camera
+// rays take 11.6 ms with eight cursors instead of 10.7, 9.5 M 6.70 instead of 6.50.
+constexpr uint32_t CURSORS_MIN_RAYS = 1u << 20, CURSORS_MAX_RAYS = 1u << 23;
+
 // Launches the persistent trace kernel over at most n_max rays (the actual count is *count_ptr
-// when given). `work` must be zero on entry, or is cleared here (clear_work).
+// when given). `work` must be zero on entry (one word), or is cleared here (clear_work: CURSOR_WORDS of
+// them).
 template <bool COUNT, class Src, class Sink, bool ANY, int W, bool SHARE>
 hipError_t launch_trace_variant(const DeviceScene& s, const TraceScratch& ts, const Src& src, const Sink& sink,
                                 const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
@@ -1386,8 +1406,8 @@ hipError_t launch_trace_variant(const DeviceScene& s, const TraceScratch& ts, co
     if (uint64_t(g) * TRACE_BLOCK > ts.threads) g = int(ts.threads / TRACE_BLOCK);
     if (g <= 0) return hipErrorInvalidValue;
     // a launch that owns all its rays statically never reads the cursor
-    if (clear_work && !(SHARE && uint64_t(n_max) <= uint64_t(g) * TRACE_BLOCK))
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, work, 1u);
+    if (clear_work && !(SHARE && !Src::CURSORS && uint64_t(n_max) <= uint64_t(g) * TRACE_BLOCK))
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(CURSOR_WORDS), 0, st, work, CURSOR_WORDS);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_trace<COUNT, Src, Sink, ANY, W, SHARE>), dim3(g), dim3(TRACE_BLOCK), 0, st, s, src,
                        sink, count_ptr, n_max, work, mask, ts, counters);
     return hipGetLastError();
@@ -1397,7 +1417,7 @@ hipError_t launch_trace_width(const DeviceScene& s, const TraceScratch& ts, cons
                               const uint32_t* count_ptr, uint32_t n_max, uint32_t* work, uint32_t mask,
                               unsigned long long* counters, hipStream_t st, bool clear_work) {
     if constexpr (!COUNT) { // the counting kernels count each ray's own traversal
-        if (n_max <= (std::is_same<Src, SrcRays>::value ? SHARE_MAX_CALLER_RAYS : SHARE_MAX_RAYS))
+        if (n_max <= (std::is_base_of<SrcRays, Src>::value ? SHARE_MAX_CALLER_RAYS : SHARE_MAX_RAYS))
             return launch_trace_variant<COUNT, Src, Sink, ANY, W, true>(s, ts, src, sink, count_ptr, n_max, work, mask,
                                                                         counters, st, clear_work);
     }
@@ -1510,6 +1530,9 @@ hipError_t launch_trace_rays(const DeviceScene& s, const TraceScratch& ts, const
     if (counters)
         return launch_trace<true>(s, ts, SrcRays{rays}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu, counters,
                                   st, true);
+    if (n >= CURSORS_MIN_RAYS && n <= CURSORS_MAX_RAYS)
+        return launch_trace<false>(s, ts, SrcSomeRays{{rays}}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu,
+                                   nullptr, st, true);
     return launch_trace<false>(s, ts, SrcRays{rays}, SinkHits{hits}, nullptr, uint32_t(n), ts.work, 0xFFu, nullptr, st,
                                true);
 }

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "bvh.h"
+#include "ray_claims.h"
 #include "../../include/merian_amd.h"
 
 namespace mrt {
@@ -73,7 +74,7 @@ constexpr int TRACE_BLOCK = 128;
 constexpr uint32_t TRACE_SPREAD = 8;
 
 // Per-context scratch of the trace kernels: the global part of the traversal stacks (`entries`
-// per thread, `threads` columns) and a ray cursor for launches that do not bring their own.
+// per thread, `threads` columns) and ray cursors (CURSOR_WORDS) for launches that do not bring their own.
 struct TraceScratch {
     uint32_t* ovf;
     uint32_t threads;

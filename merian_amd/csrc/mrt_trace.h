@@ -462,14 +462,16 @@ __device__ __forceinline__ void share_hit(WaveShared& ws, RayState& r, uint32_t 
 // when its ray is done, hands the hit to `sink` and later takes a fresh ray from `src`, so lanes
 // with short rays do not idle while others finish long ones.
 //
-// Ray indices are handed out in wave-private chunks, so the single device-wide cursor `work`
-// (zero at launch) sees a few atomics per wave instead of one per refill (it takes 117 M a second):
-// every wave first owns a static chunk of n / (2 * waves) rays (rounded down to whole waves of 64),
-// then claims guided chunks of (unclaimed rays) / (2 * waves), 64..1024 rays, from `work`. A SHARE
-// launch has so few rays per wave that the claims would be its longest part: seven eighths of its
-// rays are owned, in batches of 64 that go round the waves (neighbouring camera rays cost alike: a
-// contiguous range per wave makes the 1080p GBuffer pass 566 us instead of 440), and with at most
-// 64 rays per wave all are, evenly.
+// Ray indices are handed out in wave-private chunks, so the cursor `work` (zero at launch) sees a few
+// atomics per wave instead of one per refill (it takes 75 to 120 M a second): every wave first owns a
+// static chunk of n / (2 * waves) rays (rounded down to whole waves of 64), then claims guided chunks
+// of (unclaimed rays) / (2 * waves), 64..1024 rays, from `work`. A SHARE launch has so few rays per
+// wave that the claims would be its longest part: seven eighths of its rays are owned, in batches of
+// 64 that go round the waves (neighbouring camera rays cost alike: a contiguous range per wave makes
+// the 1080p GBuffer pass 566 us instead of 440), and with at most 64 rays per wave all are, evenly.
+//
+// Src::CURSORS: the rays are halved as without SHARE, with a cursor per 1/8 of them (ray_claims.h).
+//
 // Refilled lanes issue their ray loads before the still-active lanes' traversal step, so both
 // wait on one memory round trip.
 //
@@ -487,21 +489,27 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
     const uint32_t lane = __lane_id();
     const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    uint32_t pool, pool_end, dyn0; // dynamic claims start at dyn0
+    RayClaims claims = one_cursor(n, wave, waves);
+    uint32_t pool, pool_end, dyn0; // positions of the share (claim_ray); dynamic claims start at dyn0
     uint32_t batches = 0, batch = 0; // SHARE: batches of 64 rays this wave owns, taken so far
-    if (SHARE && n <= 64u * uint64_t(waves)) {
+    if (SHARE && !Src::CURSORS && n <= 64u * uint64_t(waves)) {
         const uint32_t each = (n + waves - 1u) / waves;
         pool = uint32_t(min(uint64_t(wave) * each, uint64_t(n)));
         pool_end = min(pool + each, n);
         dyn0 = n;
-    } else if (SHARE) {
+    } else if (SHARE && !Src::CURSORS) {
         batches = uint32_t(uint64_t(n) * 7u / (uint64_t(waves) * (8u * 64u)));
         dyn0 = batches * waves * 64u;
         pool = pool_end = 0u;
     } else {
-        const uint32_t c0 = (n / (2u * waves)) & ~63u;
-        dyn0 = c0 * waves; // <= n / 2
-        pool = wave * c0;
+        if constexpr (Src::CURSORS) {
+            claims = many_cursors(n, blockIdx.x, gridDim.x, threadIdx.x >> 6, blockDim.x >> 6);
+            work += claims.home * CURSOR_STRIDE;
+            n = claims.n;
+        }
+        const uint32_t c0 = (n / (2u * claims.waves)) & ~63u;
+        dyn0 = c0 * claims.waves; // <= n / 2
+        pool = claims.wave * c0;
         pool_end = pool + c0;
     }
     uint32_t seen = dyn0;
@@ -579,7 +587,7 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
                 batch++;
             } else if (avail < nidle && !claims_done) {
                 const uint32_t left = n - (seen < n ? seen : n);
-                const uint32_t chunk = min(max((left / (2u * waves)) & ~63u, 64u), 1024u);
+                const uint32_t chunk = min(max((left / (2u * claims.waves)) & ~63u, 64u), 1024u);
                 const uint32_t leader = uint32_t(__ffsll((unsigned long long)idle) - 1);
                 uint32_t got = 0;
                 if (lane == leader) got = atomicAdd(work, chunk);
@@ -600,7 +608,7 @@ __device__ __forceinline__ void trace_persistent(const BVH bvh, const Src& src, 
                     my = lo + (k - avail);
                 }
                 if (my != TRAVERSAL_DONE) {
-                    idx = my;
+                    idx = Src::CURSORS ? claim_ray(claims, my) : my;
                     slot = lane;
                     src.load(idx, r.o, r.d, r.tmin, r.tmax); // this lane's state is dead until ray_begin
                     fresh = true;

@@ -1,14 +1,14 @@
 // mrt_trace_closest_noalloc_dev: closest-hit ray queries that allocate no device memory.
 //
-// The trace kernel needs scratch beyond its rays and hits: a work cursor (one word, zero at the
+// The trace kernel needs scratch beyond its rays and hits: work cursors (CURSOR_WORDS, zero at the
 // start of a launch) and the global part of every lane's traversal stack (the entries past the
 // LDS part, one column per lane of the persistent grid). mrt_trace_closest_dev takes both from
 // the context, which allocates them on first use. This variant takes them from `scratch`, a
 // fixed array in device memory that every GPU the library runs on holds until the process ends.
 //
-// Layout of `scratch` (words): [0, 64) the work cursor and padding, [64, SCRATCH_WORDS) the stack
-// overflow columns: entry k of lane t at 64 + k * threads + t, for threads lanes and `entries`
-// entries per lane, threads * entries <= SCRATCH_WORDS - 64. The grid is capped at `threads`
+// Layout of `scratch` (words): [0, CURSOR_WORDS) the work cursors, [CURSOR_WORDS, SCRATCH_WORDS) the
+// stack overflow columns: entry k of lane t at CURSOR_WORDS + k * threads + t, for threads lanes and
+// `entries` entries per lane, threads * entries <= SCRATCH_WORDS - CURSOR_WORDS. The grid is capped at `threads`
 // lanes, so a deep tree runs a smaller persistent grid rather than needing more memory.
 #include <hip/hip_runtime.h>
 
@@ -25,7 +25,6 @@ namespace {
 
 constexpr uint64_t SCRATCH_BYTES = uint64_t(MRT_NOALLOC_SCRATCH_BYTES);
 constexpr uint64_t SCRATCH_WORDS = SCRATCH_BYTES / 4;
-constexpr uint64_t CURSOR_WORDS = 64;
 constexpr int MAX_DEVICES = 64;
 
 // In host code `scratch` names a host-side stand-in, not the device array: device addresses
@@ -83,7 +82,7 @@ MRT_API mrt_status mrt_trace_closest_noalloc_dev(mrt_ctx* c, mrt_scene* s, const
     ts.ovf = base + CURSOR_WORDS;
     ts.threads = uint32_t(threads);
     ts.entries = uint32_t(entries);
-    // the cursor is cleared by a fill kernel inside launch_trace_rays (no memset node)
+    // the cursors are cleared by a fill kernel inside launch_trace_rays (no memset node)
     const hipError_t e = launch_trace_rays(s->ds, ts, rays, n, hits, pick_stream(c, stream));
     return e == hipSuccess ? MRT_OK : hip_fail(c, e, "trace kernel (no-alloc)");
 }

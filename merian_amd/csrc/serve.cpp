@@ -180,7 +180,7 @@ hipError_t carve_job(Slot& sl, const Job& j, const JobShape& sh) {
     if (sh.demod) b.pb.demod = static_cast<float4*>(A(16 * N));
     b.pb.capacity = P;
     b.ts.ovf = static_cast<uint32_t*>(A(uint64_t(l.threads) * std::max<uint32_t>(1, sh.stack_entries) * 4));
-    b.ts.work = static_cast<uint32_t*>(A(64));
+    b.ts.work = static_cast<uint32_t*>(A(CURSOR_WORDS * 4));
     b.ts.threads = l.threads;
     b.ts.entries = sh.stack_entries;
     const TraceScratch tuned = scene_scratch(nullptr, j.d.scene);

@@ -9,6 +9,8 @@
 #include <deque>
 #include <vector>
 
+#include "ray_claims.h"
+
 namespace mrt {
 
 // Jobs are admitted strictly in submission order: the head of the queue is admitted once a
@@ -191,7 +193,7 @@ inline JobLayout job_layout(const JobShape& s) {
     b += round256(16 * s.npix) + round256(4 * s.npix); // accumulation, signature sum
     if (s.demod) b += round256(16 * s.npix);      // demodulation albedo
     b += round256(uint64_t(l.threads) * std::max<uint32_t>(1, s.stack_entries) * 4); // stack overflow
-    b += round256(64);                            // ray cursor
+    b += round256(4 * CURSOR_WORDS);              // ray cursors
     l.bytes = b;
     l.block = size_class(b);
     return l;

@@ -128,3 +128,31 @@ def test_shared_rays_and_refill(ctx, soup, tree, refill, grid):
     for n in (17, 4097, 130_001, *([3 << 20, len(rays)] if grid == 100 else [])):
         _same(ctx.trace(ds, rays[:n]), ref[:n])
     ds.destroy()
+
+
+@pytest.mark.parametrize("tree", [(4, 2, 0), (8, 2, 0), (8, 4, 1)])
+@pytest.mark.parametrize("grid", [100, 3, 1])
+def test_ray_counts_around_the_cursors(ctx, soup, tree, grid):
+    """Arrays on both sides of the limits of the several cursors, 2^20 and 2^23 rays, with grids that make
+    many, few and no whole rounds of them. The first 3.1 M rays against the oracle; longer arrays repeat
+    them and repeat their hits."""
+    import torch
+    pos, idx, rays, ref = soup
+    ds = _scene(ctx, pos, idx, tree)
+    t = ds.tuning()
+    t.grid_percent = grid
+    ds.set_tuning(t)
+    for n in (54_785, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 1_310_721, 2_097_153, 3 << 20, (3 << 20) + 64):
+        _same(ctx.trace(ds, rays[:n]), ref[:n])
+    if grid == 100:
+        one = torch.from_numpy(rays.view(np.float32).reshape(-1, 8)).cuda()
+        d_rays = torch.cat([one, one, one])[:(1 << 23) + 1].contiguous()
+        want = torch.from_numpy(ctx.trace(ds, rays).view(np.int32).reshape(-1, 4)).cuda()
+        want = torch.cat([want, want, want])[:len(d_rays)]
+        for n in ((1 << 23) - 1023, 1 << 23, (1 << 23) + 1):
+            got = torch.full((len(d_rays), 4), -2, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            ctx.trace_dev(ds, d_rays.data_ptr(), n, got.data_ptr(), stream=torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            assert torch.equal(got[:n], want[:n]) and bool((got[n:] == -2).all())
+    ds.destroy()
