@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from merian_amd import abi, scenes
-from merian_amd.runtime import pt_params
+from merian_amd.runtime import Guide, guide_config, pt_params
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -176,31 +176,49 @@ def test_frame_split_into_passes(ctx, small):
     _compare(split, sig2, ref, ref_sig)
 
 
-@pytest.mark.parametrize("mode", [abi.MODE_BSDF, abi.MODE_NEE])
-def test_wide_shading_tiles_match_narrow(ctx, small, mode):
-    # passes of 2^23 paths or more shade wider tiles (three paths per thread instead of two);
-    # nothing else depends on the pass size, so a frame run as one pass of 8.4 M paths equals
-    # the same frame in two passes of 4.2 M bit for bit
-    sc, ds, osc = small
+@pytest.mark.parametrize("mode", [abi.MODE_BSDF, abi.MODE_NEE, abi.MODE_GUIDED])
+@pytest.mark.parametrize("coated", [True, False])
+def test_wide_shading_tiles_match_narrow(ctx, coated, mode):
+    # scenes with a coat or sheen lobe shade wider tiles in passes of 2^23 paths or more (three paths
+    # per thread instead of two); nothing else depends on the pass size, so a frame run as one pass
+    # of 8.4 M paths equals the same frame in two passes of 4.2 M bit for bit (other scenes too)
+    import torch
+    sc = scenes.plain_small(seed=0)
+    if coated:
+        worn = np.arange(len(sc.materials)) % 3 != 0
+        sc.materials["features"][worn] |= abi.PBR_CLEARCOAT | abi.PBR_SHEEN
+        for k, v in (("coat_weight", 0.6), ("coat_alpha", 0.05), ("sheen_weight", 0.3), ("sheen_alpha", 0.2),
+                     ("sheen_color", (0.8, 0.7, 0.9))):
+            sc.materials[k][worn] = v
+    ds = ctx.scene(sc)
     W = H = 1024
     cam = ctx.camera(sc.camera, 9)
-    p = pt_params(spp=8, max_path_length=4, mode=mode)
-    t = ds.tuning()
-    saved = t.max_paths
+    p = pt_params(spp=8, max_path_length=4, mode=mode, record_signature=mode != abi.MODE_GUIDED)
+    guide = Guide(ctx, ds, guide_config(seed=3)) if mode == abi.MODE_GUIDED else None
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def frame(max_paths):
+        t = ds.tuning()
+        t.max_paths = max_paths
+        ds.set_tuning(t)
+        if guide is None:
+            img, sig, _, st = ctx.render(ds, p, cam, 9, W, H)
+            return img.tobytes(), sig.tobytes(), int(st.continuation_segments)
+        gb = torch.zeros(W * H, 4, dtype=torch.int32, device="cuda")
+        out = torch.zeros(W * H, 4, dtype=torch.float32, device="cuda")
+        ctx.gbuffer_dev(ds, cam, W, H, gb.data_ptr(), stream=stream)
+        st = guide.render_dev(ds, p, cam, 9, W, H, gb.data_ptr(), out.data_ptr(), train=False, stats=True, stream=stream)
+        torch.cuda.synchronize()
+        return out.cpu().numpy().tobytes(), b"", int(st.continuation_segments)
+
     try:
-        t.max_paths = 8 * W * H
-        ds.set_tuning(t)
-        wide, sig1, _, st1 = ctx.render(ds, p, cam, 9, W, H)
-        t = ds.tuning()
-        t.max_paths = 4 * W * H
-        ds.set_tuning(t)
-        narrow, sig2, _, st2 = ctx.render(ds, p, cam, 9, W, H)
+        wide, narrow = frame(8 * W * H), frame(4 * W * H)
     finally:
-        t = ds.tuning()
-        t.max_paths = saved
-        ds.set_tuning(t)
-    assert int(st1.continuation_segments) == int(st2.continuation_segments) > 0
-    assert wide.tobytes() == narrow.tobytes() and sig1.tobytes() == sig2.tobytes()
+        if guide is not None:
+            guide.close()
+        ds.destroy()
+    assert wide[2] == narrow[2] > 0
+    assert wide == narrow
 
 
 @pytest.mark.parametrize("which", ["default", "side"])
