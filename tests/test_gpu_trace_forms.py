@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from merian_amd import abi, scenes
+from merian_amd.runtime import pt_params
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -156,3 +157,60 @@ def test_ray_counts_around_the_cursors(ctx, soup, tree, grid):
             torch.cuda.synchronize()
             assert torch.equal(got[:n], want[:n]) and bool((got[n:] == -2).all())
     ds.destroy()
+
+
+@pytest.fixture(scope="module")
+def room():
+    return scenes.full_scene(seed=4, instances=12, env_size=(64, 32), name="room")
+
+
+@pytest.mark.parametrize("tree", [(4, 4, 0), (8, 2, 0), (8, 2, 1)])
+@pytest.mark.parametrize("w,h", [(2053, 2051), (2047, 2049), (701, 503)])
+def test_gbuffer_matches_ray_queries(ctx, room, tree, w, h):
+    """GBuffer passes above and below the 2^22 rays up to which lanes share rays, every pixel against the
+    closest hit of its camera ray (another kernel): the packed record bit for bit."""
+    import torch
+    ds = ctx.scene(room)
+    t = ds.tuning()
+    t.bvh_width, t.bvh_max_leaf, t.bvh8_order = tree
+    ds.set_tuning(t)
+    cam = ctx.camera(room.camera, 3)
+    rays, hits = (torch.zeros(w * h, k, device="cuda") for k in (8, 4))
+    gb = torch.full((w * h, 4), -2, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    ctx.camera_rays_dev(cam, w, h, rays.data_ptr(), stream=stream)
+    ctx.trace_dev(ds, rays.data_ptr(), w * h, hits.data_ptr(), stream=stream)
+    ctx.gbuffer_dev(ds, cam, w, h, gb.data_ptr(), stream=stream)
+    torch.cuda.synchronize()
+    ds.destroy()
+    got, hits = gb.cpu().numpy().view(np.uint32), hits.cpu().numpy()
+    tri = hits[:, 0].copy().view(np.uint32)
+    hit = tri != 0xFFFFFFFF
+    first = np.concatenate([[0], np.cumsum(room.geometries["primitive_count"].astype(np.int64))])
+    geom = np.searchsorted(first, tri.astype(np.int64), side="right") - 1
+    uv = hits[:, 2:4].astype(np.float16).view(np.uint16).astype(np.uint32)
+    want = np.empty_like(got)
+    want[:, :3], want[:, 3] = 0xFFFFFFFF, 0
+    want[hit, 0], want[hit, 1], want[hit, 2] = 0, (tri - first[np.where(hit, geom, 0)])[hit], geom[hit]
+    want[hit, 3] = (uv[:, 0] | uv[:, 1] << 16)[hit]
+    assert 0.2 < hit.mean() <= 1.0 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("mode", [abi.MODE_BSDF, abi.MODE_NEE])
+@pytest.mark.parametrize("tree", [(4, 4, 0), (8, 2, 0), (8, 2, 1)])
+def test_frame_of_large_passes_matches_small(ctx, room, tree, mode):
+    """Passes above the 2^22 paths up to which lanes share rays (path and shadow queues): the frame in one
+    pass of 8.4 M paths equals the same frame in passes of 2.1 M bit for bit."""
+    ds = ctx.scene(room)
+    W = H = 1024
+    cam = ctx.camera(room.camera, 7)
+    frames = []
+    for spp in (8, 2):
+        t = ds.tuning()
+        t.bvh_width, t.bvh_max_leaf, t.bvh8_order = tree
+        t.max_paths = spp * W * H
+        ds.set_tuning(t)
+        img, sig, _, st = ctx.render(ds, pt_params(spp=8, max_path_length=4, mode=mode), cam, 7, W, H)
+        frames.append((img.tobytes(), sig.tobytes(), int(st.continuation_segments)))
+    ds.destroy()
+    assert frames[0][2] > 1 << 22 and frames[0] == frames[1]
