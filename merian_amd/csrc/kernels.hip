@@ -202,12 +202,14 @@ __device__ __forceinline__ void flush_counts(const TraversalCount& c, unsigned l
 // ANY: visibility queries (first hit ends the traversal).
 // W: traversal of the scene's tree (4: BVH4Node; 8: quantised BVH8Node, sorted entries; 9: the
 // same nodes in octant order with grouped stack entries).
-// Waves per SIMD asked of the compiler (1: no limit on registers). A path queue's BVH8 traversal fits
-// 80 registers, six waves (the 1080p frame takes 169.0 ms, 171.3 with five). Camera rays hold more
-// per ray and a wave's rays end together: the 1080p GBuffer pass takes 505 us at the four waves its
-// registers allow, 550 with five, 573 with six. A ray array's BVH4 traversal fits 72 registers, seven
-// waves (4096x4096 camera rays 10.85 ms, 11.05 with six).
+// Waves per SIMD asked of the compiler (1: no limit on registers), of the kernels whose lanes do not
+// share rays. A path queue's BVH8 traversal fits 80 registers, six waves (the 1080p frame takes 164.5
+// ms, 167.4 with five). Camera rays hold more per ray: a GBuffer pass of 3840x2160 takes 1.63 and 1.43
+// ms (2 M and 500 k triangles) with five, 1.63 and 1.45 with six, 1.67 and 1.50 at the four waves that
+// its registers allow. A ray array's BVH4 traversal fits 72 registers, seven waves (4096x4096 camera
+// rays 10.69 ms, 10.90 with six).
 template <class Src, int W> constexpr int TRACE_WAVES = W == 9 ? 5 : 1;
+template <> constexpr int TRACE_WAVES<SrcCamera, 8> = 5;
 template <> constexpr int TRACE_WAVES<SrcQueue, 8> = 6;
 template <> constexpr int TRACE_WAVES<SrcShadow, 8> = 6;
 template <> constexpr int TRACE_WAVES<SrcRays, 8> = 5;
