@@ -21,15 +21,12 @@ struct alignas(16) TriRecord {
 
 // Leaf stack entries: bit 31 set, first record in bits 3..30, (count - 1) in bits 0..2.
 constexpr uint32_t LEAF_FLAG = 0x80000000u;
-inline uint32_t leaf_entry(uint32_t first, uint32_t count) { return LEAF_FLAG | (first << 3) | (count - 1u); }
 constexpr int MAX_LEAF = 8; // most triangles per leaf the encoding allows (the build default is 4)
 
-// v0/e1/e2: per-triangle float[3] operands exactly as the intersection test uses them
-// (e1 = v1 - v0, e2 = v2 - v0 rounded in float). flags as in TriRecord.
 // 8-wide node with child boxes quantised to 8 bits on a per-node power-of-two grid (80 bytes,
-// five 16-byte loads): child box = fma(q, 2^e, origin) per plane, every decoded box containing
-// the padded child box exactly as the BVH4 stores it. Inner children are stored consecutively
-// from child_base in slot order; the triangles of the leaf children consecutively from tri_base.
+// five 16-byte loads): child box = fma(q, 2^e, origin) per plane, rounded outward, so that every
+// decoded box contains the padded child box. Inner children are stored consecutively from child_base
+// in slot order; the triangles of the leaf children consecutively from tri_base.
 // One code byte per slot makes the slot's traversal entry a select and an add:
 //   leaf:  (first triangle - tri_base) << 3 | (count - 1)   (<= BVH8_LEAF_CODE_MAX)
 //   empty: BVH8_EMPTY
@@ -90,6 +87,8 @@ inline float bvh_dir_min(int max_exp) {
     return e > -66 ? __builtin_ldexpf(1.0f, e < 126 ? e : 126) : 1e-20f;
 }
 
+// v0/e1/e2: per-triangle float[3] operands exactly as the intersection test uses them
+// (e1 = v1 - v0, e2 = v2 - v0 rounded in float). flags as in TriRecord.
 // max_leaf: most triangles per leaf (1..MAX_LEAF); traversal_cost: SAH cost of one node
 // visit relative to one triangle test.
 BVH8 build_bvh8(const float* v0, const float* e1, const float* e2, const uint32_t* flags, uint32_t n,
