@@ -50,6 +50,13 @@ def trace_variant(tuning: dict) -> int:
     return 9 if w == 8 and int(tuning.get("bvh8_order", 0)) == 1 else w
 
 
+def queue_kernel(tuning: dict, pixels: int, spp: int) -> str:
+    """Name of the intersect kernel of a frame's path queue. Its last template argument says whether
+    lanes share rays: passes of at most 2^22 paths (merian_amd/csrc/kernels.hip, SHARE_MAX_RAYS)."""
+    paths = pixels * max(1, min(spp, int(tuning["max_paths"]) // pixels))
+    return f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(tuning)}, {str(paths <= 1 << 22).lower()}>"
+
+
 def roofline(kernel: str, avg_ms: float, launches: int, algorithmic_bytes: float, profile: str,
              match: dict | None = None, extra: dict | None = None) -> dict:
     """Bandwidth roofline of one kernel. `achieved` is the HBM-side traffic per dispatch that a
@@ -59,7 +66,8 @@ def roofline(kernel: str, avg_ms: float, launches: int, algorithmic_bytes: float
     algorithmic bytes (every node, triangle and ray the traversal touches, most of them served by
     L2) stay beside it as a diagnostic. The profile applies only if it was taken with the settings
     in `match` (tuning, workload); otherwise `achieved` falls back to the algorithmic rate and says
-    so; a profile of another kernel does not apply either. Reads are scaled by what FETCH_SIZE shows for random whole-line gathers of known size
+    so, without a fraction if that is above the HBM peak (caches then serve most of it); a profile of
+    another kernel does not apply either. Reads are scaled by what FETCH_SIZE shows for random whole-line gathers of known size
     (exact: 64 bytes per request, two per 128-byte line fill); `traffic_upper` scales them by the
     copy's factor instead (streaming reads count one request per 128-byte line)."""
     alg_gbs = algorithmic_bytes / (avg_ms * 1e-3) / 1e9
@@ -98,7 +106,8 @@ def roofline(kernel: str, avg_ms: float, launches: int, algorithmic_bytes: float
             if tj.get(k) is not None:
                 r[k] = tj[k]
     else:
-        r.update({"achieved": round(alg_gbs, 1), "frac": round(alg_gbs / HBM_PEAK_GBS, 4), "traffic": None,
+        frac = round(alg_gbs / HBM_PEAK_GBS, 4)
+        r.update({"achieved": round(alg_gbs, 1), "frac": frac if frac <= 1.0 else None, "traffic": None,
                   "basis": "algorithmic bytes (no profile of this workload and tuning)"})
     if extra:
         r.update(extra)
@@ -211,7 +220,7 @@ def small_leg(ctx, frames: int = 64, retune: bool = False) -> dict:
     bytes_per_seg = (st_c.node_visits * node_bytes + st_c.triangle_tests * TRI_BYTES) / cont + RAY_IO_BYTES
     cont_timed = segs - frames * W * H
     avg_ms = ms_trace / max(1, launches)
-    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(tuning)}, true>", avg_ms, launches,
+    roof = roofline(queue_kernel(tuning, W * H, 4), avg_ms, launches,
                     bytes_per_seg * cont_timed / max(1, launches), SMALL_TRAFFIC,
                     match={"tuning": tuning, "workload": SMALL_WORKLOAD},
                     extra={"bytes_per_segment": round(bytes_per_seg, 1)})
@@ -716,8 +725,7 @@ def main():
     cont_timed = segs - args.steps * W * H
     bytes_per_launch = bytes_per_seg * cont_timed / max(1, launches)
     avg_ms = ms_trace / max(1, launches)
-    roof = roofline(f"k_trace<false, SrcQueue, SinkQueue, false, {trace_variant(ds.tuning().as_dict())}, false>", avg_ms, launches,
-                    bytes_per_launch, TRAFFIC_FILE,
+    roof = roofline(queue_kernel(ds.tuning().as_dict(), W * H, args.spp), avg_ms, launches, bytes_per_launch, TRAFFIC_FILE,
                     match={"tuning": tuning, "workload": TRAFFIC_WORKLOAD},
                     extra={"bytes_per_segment": round(bytes_per_seg, 1), "node_bytes": node_bytes,
                            "node_visits_per_segment": round(st_c.node_visits / cont, 2),

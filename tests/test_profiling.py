@@ -150,3 +150,21 @@ def test_bench_roofline_ignores_a_profile_of_another_kernel(tmp_path):
     assert bench.roofline("k_trace<..., 9>", 1.0, 10, 8e9, str(prof_json), match=m)["traffic"] is None
     assert bench.trace_variant({"bvh_width": 8, "bvh8_order": 1}) == 9 and bench.trace_variant({"bvh_width": 8}) == 8
     assert bench.trace_variant({"bvh_width": 4, "bvh8_order": 1}) == 4
+
+
+def test_bench_roofline_without_a_profile_gives_no_fraction_above_one(tmp_path):
+    sys.path.insert(0, str(ROOT))
+    import bench
+    r = bench.roofline("k", 1.0, 1, 9e9, str(tmp_path / "none.json"))
+    assert r["frac"] is None and r["traffic"] is None and r["achieved"] == 9000.0
+
+
+def test_bench_names_the_kernel_that_a_pass_runs():
+    sys.path.insert(0, str(ROOT))
+    import bench
+    k = "k_trace<false, SrcQueue, SinkQueue, false, "
+    assert bench.queue_kernel({"max_paths": 1 << 25, "bvh_width": 4}, 512 * 512, 4) == k + "4, true>"
+    assert bench.queue_kernel({"max_paths": 1 << 28, "bvh_width": 8}, 1920 * 1080, 2) == k + "8, true>"
+    assert bench.queue_kernel({"max_paths": 1 << 28, "bvh_width": 8}, 1920 * 1080, 64) == k + "8, false>"
+    # a pass holds whole samples: two of 2.07 M paths each fit 2^22
+    assert bench.queue_kernel({"max_paths": 1 << 22, "bvh_width": 8, "bvh8_order": 1}, 1920 * 1080, 64) == k + "9, true>"
