@@ -61,3 +61,32 @@ def test_noalloc_rejects_oversize_requests():
             ctx.trace_noalloc_dev(ds, 0, 0, 0)        # an empty query is a no-op
         finally:
             ds.destroy()
+
+
+@pytest.mark.parametrize("n", [300_001, (1 << 20) + 5, (3 << 20) + 77])
+def test_noalloc_trace_captured(n):
+    """Captured before any other query of its size, on one and on several work cursors, and replayed with
+    eager queries between (which leave the cursors used): every replay gives the eager hits."""
+    import torch
+    pos, idx = scenes.ray_query(seed=5, n_tri=20_000)
+    with Context(0) as ctx:
+        ds = ctx.triangles(pos, idx)
+        try:
+            sets = [torch.from_numpy(scenes.incoherent_rays(n, seed=k).view(np.uint8)).cuda() for k in (1, 2)]
+            rays, got = sets[0].clone(), torch.zeros(n * 16, dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                ctx.trace_noalloc_dev(ds, rays.data_ptr(), n, got.data_ptr(),
+                                      stream=torch.cuda.current_stream().cuda_stream)
+            ref = torch.zeros(n * 16, dtype=torch.uint8, device="cuda")
+            for k in (0, 1, 0):
+                rays.copy_(sets[k])
+                got.fill_(0xAB)
+                graph.replay()
+                torch.cuda.synchronize()
+                ctx.trace_noalloc_dev(ds, sets[k].data_ptr(), n, ref.data_ptr())
+                ctx.synchronize()
+                assert torch.equal(got, ref), f"replay of set {k}"
+        finally:
+            ds.destroy()
